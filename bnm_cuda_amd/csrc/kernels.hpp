@@ -81,6 +81,17 @@ hipError_t launch_sim_ei64(const double* SC, const SimArgs& a, int LS, hipStream
 // form: 0 as written, 1 DPP row broadcast (LS = 4, N <= 128), 2 / 3 short-chain
 // update with four / one partial sums in the coupling dot
 hipError_t launch_sim_ei(const float* SC, const SimArgs& a, int LS, int form, hipStream_t st);
+// row-blocked kernel (sim_block.hip): FP32 strict, N <= 256; FP64, N <= 128
+struct BlockShape {
+    int KC;        // k values per lane (template)
+    int SS;        // LDS slice stride (elements)
+    int threads;
+    size_t smem;
+    bool ok;
+};
+BlockShape block_shape(int N, size_t elem);
+template <class T>
+hipError_t launch_sim_block(const T* SC, const SimArgs& a, hipStream_t st);
 template <class R>
 hipError_t launch_sim_stream(const R* SCt, const SimArgs& a, int KS, hipStream_t st);
 
