@@ -420,8 +420,9 @@ static int ctx_alloc(bnm_ctx* x) {
         std::vector<int> st(x->nseg), ln(x->nseg);
         st[0] = c.n_vols_remove;
         ln[0] = x->ots - c.n_vols_remove;
-        std::vector<int> ws(x->nw > 0 ? x->nw : 1), we(x->nw > 0 ? x->nw : 1);
-        bnm_window_bounds(&c, ws.data(), we.data());
+        std::vector<int> ws(x->nw), we(x->nw);
+        // (with no_fcd nw is 0, whatever windows the configuration has)
+        if (x->nw > 0) bnm_window_bounds(&c, ws.data(), we.data());
         for (int w = 0; w + 1 < x->nseg; ++w) {
             st[w + 1] = ws[w];
             ln[w + 1] = we[w] - ws[w] + 1;

@@ -71,3 +71,19 @@ def _check(oracle_mod, prec, N, period):
     assert rel <= (1e-9 if f64 else 1e-6)
     scale = np.abs(r["ext"]).max(axis=(0, 2), keepdims=True)
     assert (np.abs(g["ext"] - r["ext"]) <= (1e-9 if f64 else 1e-5) * scale).all()
+
+
+def test_no_fcd_with_many_windows():
+    """no_fcd leaves the configuration's windows out: a context whose window
+    settings give hundreds of them keeps no window tables, and FC and cost are
+    those of the same run without a window that fits."""
+    N, prec = 12, bnm.PREC_F64
+    SC, G, wEE, wEI, noise, emp_fc, emp_fcd = _case(N, T + 1, 5)
+    out = []
+    for window, step in ((4, 1), (4000, 1)):
+        cfg = bnm.default_config(nodes=N, n_sims=B, time_steps=T, bold_tr=5, n_vols_remove=2, window_size=window,
+                                 window_step=step, exc_interhemispheric=0, noise_period_ms=T + 1, adjust_fic=0,
+                                 no_fcd=1, precision=prec, kernel=bnm.KERNEL_FAST)
+        out.append(bnm.run_simulations(cfg, SC, G, wEE, wEI, noise=noise, emp_fc=emp_fc, emp_fcd=emp_fcd))
+    np.testing.assert_array_equal(out[0]["fc"], out[1]["fc"])
+    np.testing.assert_array_equal(out[0]["corr"], out[1]["corr"])
