@@ -68,7 +68,8 @@ struct Variant {
                 // 7 FP64 stream with register/LDS-resident SC,
                 // 5 stream with register/LDS-resident SC (FP32; mode 1: S_E by
                 //   DPP row broadcast, 2: and three streamed chunks in flight),
-                // 8 sparse row lists, 9 row-blocked
+                // 8 sparse row lists, 9 row-blocked,
+                // 10 several workgroups per simulation
     int ls, ks, mode;
 };
 
@@ -137,9 +138,15 @@ struct bnm_ctx {
     std::string kname = "none";
     std::string tune_log;
     bool tuned = false;
-    double ms_per_sim_ms = -1;   // integration time per simulated ms of the chosen variant (tuner)
     int autotune = 1, tune_ms = 300;
     Variant variant{0, 4, 1, 0};
+    // the best variant with one workgroup per simulation: what a graph of several
+    // contexts runs (its branches fill the CUs), and what runs the simulations
+    // whose workgroups did not find each other
+    Variant solo{0, 4, 1, 0};
+    double solo_ms_per_sim_ms = -1;
+    unsigned long long* gang = nullptr;   // exchange words of kind 10
+    int gang_mode = -1, gang_polls = kGangStartPolls;
     hipGraphExec_t graph_exec = nullptr;
     bool have_sc = false, have_noise = false, have_emp = false, have_params = false;
     int fast_ls = 0, fast_ks = 0, stream_ks = 0, force_stream = 0, no_ei = 0, ei_ls = 0, ei_bc = 0, ei_form = -1, no_hyb = 0, hyb_ks = 0, hyb_bc = -1, hyb_rr = -1;
@@ -359,7 +366,7 @@ int bnm_make_noise_chunked(unsigned seed, long long count, float* out, int threa
 
 void bnm_ctx_destroy(bnm_ctx* x) {
     if (!x) return;
-    void* bufs[] = {x->SC64, x->SC32, x->SCt64, x->SCt32, x->SCc32, x->SCc64, x->SPw[0], x->SPw[1], x->SPw64[0], x->SPw64[1], x->SPd[0], x->SPd[1], x->noise, x->G, x->wEE, x->wEI, x->wIE, x->wIEfic,
+    void* bufs[] = {x->SC64, x->SC32, x->SCt64, x->SCt32, x->SCc32, x->SCc64, x->SPw[0], x->SPw[1], x->SPw64[0], x->SPw64[1], x->SPd[0], x->SPd[1], x->gang, x->noise, x->G, x->wEE, x->wEI, x->wIE, x->wIEfic,
                     x->wIEadj, x->wIEscratch, x->bold, x->ext, x->failed, x->trials, x->unstable,
                     x->seg_start, x->seg_len, x->pidx, x->mean, x->inv, x->wmean, x->winv, x->fc,
                     x->wfc, x->wz, x->wzlo, x->fcd, x->emp_c, x->ks_u, x->ks_fe, x->bins, x->nanf, x->corr, x->pen,
@@ -402,6 +409,7 @@ static int ctx_alloc(bnm_ctx* x) {
         }
         if ((r = cdalloc(x, &x->SPd[i], (size_t)(kSparseRW + kSparseLL) / 4 * ls * N))) return r;
     }
+    if (!x->arena && gang_shape(x->N, rsz).ok && (r = cdalloc(x, &x->gang, gang_words(x->N, x->B, rsz)))) return r;
     if ((r = cdalloc(x, &x->G, B))) return r;
     if ((r = cdalloc(x, &x->wEE, B * N))) return r;
     if ((r = cdalloc(x, &x->wEI, B * N))) return r;
@@ -594,6 +602,12 @@ static bnm_ctx* ctx_create(const bnm_config* cfg, int* status, unsigned char* ar
     // BNM_SPARSE_STRICT=0: the sparse kernel with the plain FP32 node update
     // instead of the strict one (the default)
     x->sparse_mode = env_int("BNM_SPARSE_STRICT", 1) ? 64 : 0;
+    // BNM_GANG: 1 pins the kernel with several workgroups per simulation where it
+    // applies, 0 leaves it out; BNM_GANG_POLLS: how long a workgroup waits for
+    // the others of its simulation (-1: not at all, every simulation then runs on
+    // one workgroup)
+    x->gang_mode = env_int("BNM_GANG", -1);
+    x->gang_polls = env_int("BNM_GANG_POLLS", kGangStartPolls);
     x->hyb_ks = env_int("BNM_HYB_KS", 0);
     {
         int dev = 0, v = 0;
@@ -789,6 +803,7 @@ static bool variant_ok(const bnm_ctx* x, const Variant& v) {
             return (v.ls == 1 || v.ls == 2) && x->sp_P[v.ls - 1] > 0 && !(x->f64 && (v.mode & 64)) &&
                    sparse_shape(x->N, x->sp_P[v.ls - 1], v.ls, x->lds_max, el).ok;
         case 9: return block_shape(x->N, el).ok;
+        case 10: return x->gang && gang_shape(x->N, el).ok;
         default: return true;
     }
 }
@@ -822,6 +837,10 @@ static std::string variant_name(const bnm_ctx* x, const Variant& v) {
     } else if (v.kind == 9) {
         const BlockShape g = block_shape(x->N, el);
         std::snprintf(name, sizeof name, "block_%s(R=4,KC=%d,threads=%d%s)", p, g.KC, g.threads,
+                      x->f64 ? "" : ",strict");
+    } else if (v.kind == 10) {
+        const GangShape g = gang_shape(x->N, el);
+        std::snprintf(name, sizeof name, "gang_%s(C=%d,R=%d,KC=%d,threads=%d%s)", p, g.C, g.R, g.KC, kGangThreads,
                       x->f64 ? "" : ",strict");
     } else if (v.kind == 7) {
         const FastShape g = hyb64_shape(x->N, v.ks, x->lds_max, x->hyb_rr);
@@ -863,6 +882,14 @@ static hipError_t launch_variant(bnm_ctx* x, const Variant& v, const SimArgs& a,
             return launch_sim_sparse(x->SPw[v.ls - 1], x->SPd[v.ls - 1], a, x->sp_P[v.ls - 1], v.ls, (v.mode & 64) != 0,
                                      x->lds_max, st);
         case 9: return x->f64 ? launch_sim_block<double>(x->SC64, a, st) : launch_sim_block<float>(x->SC32, a, st);
+        case 10: {
+            const hipError_t e = x->f64 ? launch_sim_gang<double>(x->SC64, a, x->gang, x->gang_polls, st)
+                                        : launch_sim_gang<float>(x->SC32, a, x->gang, x->gang_polls, st);
+            if (e != hipSuccess) return e;
+            SimArgs b = a;
+            b.only = gang_state(x->gang, x->N, x->B, x->f64 ? 8 : 4);
+            return launch_variant(x, x->solo, b, st);
+        }
         default:
             return x->f64 ? launch_sim_plain<double>(x->SC64, a, st)
                           : launch_sim_plain<float>(x->SC32, a, st);
@@ -973,6 +1000,18 @@ static std::vector<Variant> candidates(const bnm_ctx* x) {
             add({8, 2, 1, spm});
         }
     }
+    // several workgroups per simulation: where it pays depends on the population
+    // (N = 400, FP32: 0.7 us a substep on seven CUs against 2.6 on one), so it
+    // is for the tuner to say
+    if (c.kernel == BNM_KERNEL_AUTO && (x->autotune || x->gang_mode > 0) && !switched) {
+        // (the tuner's order: what is likely best first, see choose_variant; the
+        // streaming kernels are left out where a hybrid one applies)
+        bool hyb = false;
+        for (const Variant& v : out) hyb = hyb || v.kind == 5 || v.kind == 7;
+        if (hyb) out.erase(std::remove_if(out.begin(), out.end(), [](const Variant& v) { return v.kind == 1; }), out.end());
+        std::stable_partition(out.begin(), out.end(), [](const Variant& v) { return v.kind == 8; });
+        if (x->gang_mode != 0) add({10, 1, 1, 0});
+    }
     // the MFMA kernel implements FP32 too; the tuner may pick it for large populations
     if (c.kernel == BNM_KERNEL_AUTO && !x->f64 && !pinned && !x->force_stream) add({2, 0, 0, 0});
     return out;
@@ -1018,9 +1057,12 @@ static int choose_variant(bnm_ctx* x) {
     if (x->tuned) return BNM_OK;
     std::vector<Variant> cs = candidates(x);
     if (cs.empty()) return fail(BNM_E_UNSUP, "no integration kernel fits this configuration");
-    x->variant = cs[0];
+    x->variant = x->solo = cs[0];
+    x->solo_ms_per_sim_ms = -1;
     x->tune_log.clear();
-    if (cs.size() > 1 && x->cfg.kernel == BNM_KERNEL_AUTO && x->autotune) {
+    if (x->gang_mode > 0 && cs.back().kind == 10) {
+        x->variant = cs.back();
+    } else if (cs.size() > 1 && x->cfg.kernel == BNM_KERNEL_AUTO && x->autotune) {
         SimArgs a = make_args(x);
         a.time_steps = std::min(x->cfg.time_steps, x->tune_ms);
         a.adjust_fic = 0;
@@ -1041,9 +1083,15 @@ static int choose_variant(bnm_ctx* x) {
             std::snprintf(buf, sizeof buf, "%s%s=%.3fms", x->tune_log.empty() ? "" : "; ",
                           variant_name(x, v).c_str(), mn);
             x->tune_log += buf;
-            if (mn < best) { best = mn; x->variant = v; }
+            if (mn < best) {
+                best = mn;
+                x->variant = v;
+                if (v.kind != 10) {   // (kind 10 comes last)
+                    x->solo = v;
+                    x->solo_ms_per_sim_ms = best / std::max(1, (int)a.time_steps + 1);
+                }
+            }
         }
-        x->ms_per_sim_ms = best / std::max(1, (int)a.time_steps + 1);
     }
     x->kname = variant_name(x, x->variant);
     x->tuned = true;
@@ -1054,7 +1102,8 @@ static int choose_variant(bnm_ctx* x) {
 // recorded (not inside graph capture).
 // analyze_only: FC, FCD and fit of the BOLD already in the context (no FIC
 // initialisation, no integration, no FIC penalty)
-static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only = false) {
+// solo: with one workgroup per simulation (several contexts in one graph)
+static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only = false, bool solo = false) {
     const bnm_config& c = x->cfg;
     if (timed) HIPCHK(hipEventRecord(x->ev[0], st));
     if (c.do_fic && c.analytical_fic && !analyze_only)
@@ -1063,7 +1112,7 @@ static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only
     if (timed) HIPCHK(hipEventRecord(x->ev[1], st));
     if (!analyze_only) {
         const SimArgs a = make_args(x);
-        HIPCHK(launch_variant(x, x->variant, a, st));
+        HIPCHK(launch_variant(x, solo ? x->solo : x->variant, a, st));
     }
     if (timed) HIPCHK(hipEventRecord(x->ev[2], st));
     if (!c.sim_only) {
@@ -1286,26 +1335,27 @@ struct bnm_multi {
 // simulated ms, or one timed window of the chosen variant when the tuner did
 // not time it, times the run's simulated ms (FIC restarts not included).
 static int estimate_ms(bnm_ctx* x, double* out) {
-    if (x->ms_per_sim_ms < 0) {
+    double& per = x->solo_ms_per_sim_ms;
+    if (per < 0) {
         SimArgs a = make_args(x);
         a.time_steps = std::min(x->cfg.time_steps, x->tune_ms);
         a.adjust_fic = 0;
         a.wIE_out = x->wIEscratch;
         float ms = 0;
         HIPCHK(hipEventRecord(x->ev[0], x->st));
-        HIPCHK(launch_variant(x, x->variant, a, x->st));
+        HIPCHK(launch_variant(x, x->solo, a, x->st));
         HIPCHK(hipEventRecord(x->ev[1], x->st));
         HIPCHK(hipEventSynchronize(x->ev[1]));
         HIPCHK(hipEventElapsedTime(&ms, x->ev[0], x->ev[1]));
-        x->ms_per_sim_ms = ms / std::max(1, (int)a.time_steps + 1);
+        per = ms / std::max(1, (int)a.time_steps + 1);
     }
-    *out = x->ms_per_sim_ms * (x->cfg.time_steps + 1);
+    *out = per * (x->cfg.time_steps + 1);
     return BNM_OK;
 }
 
 // workgroups of the context's integration kernel (one per simulation, or one
 // per 16 for the MFMA kernel)
-static int integration_wgs(const bnm_ctx* x) { return x->variant.kind == 2 ? (x->B + 15) / 16 : x->B; }
+static int integration_wgs(const bnm_ctx* x) { return x->solo.kind == 2 ? (x->B + 15) / 16 : x->B; }
 
 // A "small" integration workgroup: at most 4 waves and 32 KB of LDS.  Two
 // such workgroups of different kernels always fit one CU together (8 waves,
@@ -1313,7 +1363,7 @@ static int integration_wgs(const bnm_ctx* x) { return x->variant.kind == 2 ? (x-
 // runs about as fast beside another as alone (two 256-thread E/I workgroups
 // per CU take the time of one).
 static bool small_workgroup(const bnm_ctx* x) {
-    const Variant& v = x->variant;
+    const Variant& v = x->solo;
     const size_t el = x->f64 ? 8 : 4;
     int threads = 1024;
     size_t smem = 0;
@@ -1447,7 +1497,7 @@ bnm_multi* bnm_multi_create(bnm_ctx** ctxs, int n, int* status) {
         for (const auto& st : stages[b]) {
             if (r || e != hipSuccess) break;
             if (st.size() == 1) {
-                r = enqueue_run(m->ctxs[st[0]], bst[b], false);
+                r = enqueue_run(m->ctxs[st[0]], bst[b], false, false, true);
                 continue;
             }
             // the second context on its own stream, forked from and joined to
@@ -1460,8 +1510,8 @@ bnm_multi* bnm_multi_create(bnm_ctx** ctxs, int n, int* status) {
             hipStream_t s2 = m->ctxs[st[1]]->st;
             if (e == hipSuccess) e = hipEventRecord(f, bst[b]);
             if (e == hipSuccess) e = hipStreamWaitEvent(s2, f, 0);
-            if (e == hipSuccess) r = enqueue_run(m->ctxs[st[0]], bst[b], false);
-            if (e == hipSuccess && !r) r = enqueue_run(m->ctxs[st[1]], s2, false);
+            if (e == hipSuccess) r = enqueue_run(m->ctxs[st[0]], bst[b], false, false, true);
+            if (e == hipSuccess && !r) r = enqueue_run(m->ctxs[st[1]], s2, false, false, true);
             if (e == hipSuccess && !r) e = hipEventRecord(jn, s2);
             if (e == hipSuccess && !r) e = hipStreamWaitEvent(bst[b], jn, 0);
         }
