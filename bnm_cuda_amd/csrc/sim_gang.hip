@@ -29,10 +29,15 @@
 // time loop end when the others get there; they have a bound too (kLoopPolls),
 // with the same consequence.
 //
-// What bounds it: the exchange.  One substep is about 1000 cycles of store to
-// poll, 400 of FMAs, 250 of sums, update and LDS; against the sparse kernel on
-// one CU (6330 cycles at N = 400 / 40 %), which walks its row with an add, a
-// gather and an FMA per nonzero.
+// What bounds it: the exchange.  At N = 400 (FP32, 16 simulations on 112 CUs) one
+// substep is 1810 cycles: 850 from store to the value in the others' LDS, 450 of
+// FMAs (100 a lane) and LDS reads, 160 of update, the rest sums, barrier and BW;
+// the sparse kernel on one CU, which walks its row with an add, a gather and an
+// FMA per nonzero, takes 6330 (40 % dense).  FP64, N = 200 (32 simulations on 128
+// CUs): 2030 against the sparse kernel's 3020 (33 % dense) and the hybrid's 11660.
+// Polling with two loads in flight, or with pauses, is no faster (1980, 1760 to
+// 1880 cycles).  LDS-resident S has to be 16-byte aligned: behind the three
+// flags without it every 16-byte read took several times as long (3060 cycles).
 #include <algorithm>
 #include <type_traits>
 
@@ -270,54 +275,55 @@ __global__ __launch_bounds__(kGangThreads) void k_sim_gang(const T* __restrict__
 #pragma unroll
         for (int s = 0; s < 10; ++s) {
             ++seq;
-            {
-                const T* Sx = Sr + (s & 1) * ldS;
-                T v[KC];
+            // the next millisecond's draw, ahead of the store that the others wait for
+            // (behind it: 2030 cycles a substep against 1810)
+            const float drawn = s < 9 ? draw(ms1, s + 1) : draw(ms2, 0);
+            const T* Sx = Sr + (s & 1) * ldS;
+            T v[KC];
 #pragma unroll
-                for (int i = 0; i + VW <= KC; i += VW) {
-                    const vec t = *reinterpret_cast<const vec*>(Sx + i);
+            for (int i = 0; i + VW <= KC; i += VW) {
+                const vec t = *reinterpret_cast<const vec*>(Sx + i);
 #pragma unroll
-                    for (int w = 0; w < VW; ++w) v[i + w] = t[w];
-                }
+                for (int w = 0; w < VW; ++w) v[i + w] = t[w];
+            }
 #pragma unroll
-                for (int i = KC / VW * VW; i < KC; ++i) v[i] = Sx[i];
-                T acc[R];
+            for (int i = KC / VW * VW; i < KC; ++i) v[i] = Sx[i];
+            T acc[R];
 #pragma unroll
-                for (int r = 0; r < R; ++r) acc[r] = sc[r][0] * v[0];
+            for (int r = 0; r < R; ++r) acc[r] = sc[r][0] * v[0];
 #pragma unroll
-                for (int i = 1; i < KC; ++i)
+            for (int i = 1; i < KC; ++i)
 #pragma unroll
-                    for (int r = 0; r < R; ++r) acc[r] = fma(sc[r][i], v[i], acc[r]);
-                const T c = gang_sum(acc);
-                p.after(c, s == 9);
-                if constexpr (F64) {
-                    const u64 u = __double_as_longlong(p.S);
-                    __builtin_amdgcn_raw_buffer_store_b128(u32x4{(unsigned)u, seq, (unsigned)(u >> 32), seq}, xr, xput,
-                                                           ((s + 1) & 1) * xrow, 0);
-                } else {
-                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(p.S), seq}, xr, xput,
-                                                          ((s + 1) & 1) * xrow, 0);
-                }
-                Sb[(s & 1) ? own : own1] = p.S;
-                // while the words are on their way
-                p.settle();
-                if (s < 9) {
-                    p.before(nz[s + 1]);
-                    nz[s + 1] = draw(ms1, s + 1);
-                } else {
-                    p.before(nz[0]);
-                    nz[0] = draw(ms2, 0);
-                }
-                if constexpr (F64) {
-                    if (s == 9 && writer) bw.step(p.S);
-                } else {
-                    if (s == 1) bw.template part<0>(bwS);
-                    if (s == 2) bw.template part<1>(bwS);
-                    if (s == 3) bw.template part<2>(bwS);
-                    if (s == 4) bw.template part<3>(bwS);
-                    if (s == 5) bw.template part<4>(bwS);
-                    if (s == 6) bw.template part<5>(bwS);
-                }
+                for (int r = 0; r < R; ++r) acc[r] = fma(sc[r][i], v[i], acc[r]);
+            const T c = gang_sum(acc);
+            p.after(c, s == 9);
+            if constexpr (F64) {
+                const u64 u = __double_as_longlong(p.S);
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4{(unsigned)u, seq, (unsigned)(u >> 32), seq}, xr, xput,
+                                                       ((s + 1) & 1) * xrow, 0);
+            } else {
+                __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(p.S), seq}, xr, xput,
+                                                      ((s + 1) & 1) * xrow, 0);
+            }
+            Sb[(s & 1) ? own : own1] = p.S;
+            // while the words are on their way
+            p.settle();
+            if (s < 9) {
+                p.before(nz[s + 1]);
+                nz[s + 1] = drawn;
+            } else {
+                p.before(nz[0]);
+                nz[0] = drawn;
+            }
+            if constexpr (F64) {
+                if (s == 9 && writer) bw.step(p.S);
+            } else {
+                if (s == 1) bw.template part<0>(bwS);
+                if (s == 2) bw.template part<1>(bwS);
+                if (s == 3) bw.template part<2>(bwS);
+                if (s == 4) bw.template part<3>(bwS);
+                if (s == 5) bw.template part<4>(bwS);
+                if (s == 6) bw.template part<5>(bwS);
             }
             lds_barrier();
         }
