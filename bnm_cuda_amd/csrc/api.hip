@@ -950,6 +950,10 @@ static std::vector<Variant> candidates(const bnm_ctx* x) {
                 add({8, 1, 1, spm});
                 add({8, 2, 1, spm});
             } else if (c.kernel == BNM_KERNEL_AUTO && !x->f64) {
+                // (large populations of few nodes are a matter of instructions per
+                // simulation, not of latency: both pools in one lane, one wave for
+                // 64 nodes, 1.17 ms against 1.62 at N = 41, 2036 simulations)
+                if (x->B > 512) add({0, 1, 1, 0});
                 add({2, 0, 0, 0});
             }
             return out;

@@ -49,8 +49,8 @@ __device__ __forceinline__ int block_row(int q, int r) {
 
 }  // namespace
 
-template <class T, int R, int KC, int MAXT>
-__global__ __launch_bounds__(MAXT) void k_sim_block(const T* __restrict__ SC, SimArgs a, int SS) {
+template <class T, int R, int KC, int MAXT, int WAVES>
+__global__ __launch_bounds__(MAXT, WAVES) void k_sim_block(const T* __restrict__ SC, SimArgs a, int SS) {
     constexpr int Q = 2 * R;                       // lanes of a group, k-slices
     constexpr int VW = 16 / sizeof(T);
     typedef T vec __attribute__((ext_vector_type(VW)));
@@ -251,10 +251,28 @@ BlockShape block_shape(int N, size_t elem) {
     return s;
 }
 
+template <class T, int KC, int WAVES>
+static void launch_block_w(const T* SC, const SimArgs& a, const BlockShape& s, hipStream_t st) {
+    constexpr int MAXT = KC <= 16 ? 256 : 512;
+    hipLaunchKernelGGL((k_sim_block<T, 4, KC, MAXT, WAVES>), dim3(a.B), dim3(s.threads), s.smem, st, SC, a, s.SS);
+}
+
+// Registers against waves (FP32, N <= 128).  With few simulations a CU the
+// substep's latency counts, with many the waves that hide it: the build for four
+// waves a SIMD (128 VGPRs, what is used once a millisecond spilled) against the
+// one without spills takes, in cycles a substep, N = 41: 527 / 537 at 128
+// simulations, 1097 / 1403 at 2048; N = 64: 555 / 575 and 1195 / 1488; N = 100:
+// 698 / 677, 844 / 822 at 512, 1436 / 1602 at 1024, 2657 / 3068 at 2048.
 template <class T, int KC>
 static void launch_block(const T* SC, const SimArgs& a, const BlockShape& s, hipStream_t st) {
-    constexpr int MAXT = KC <= 16 ? 256 : 512;
-    hipLaunchKernelGGL((k_sim_block<T, 4, KC, MAXT>), dim3(a.B), dim3(s.threads), s.smem, st, SC, a, s.SS);
+    if constexpr (sizeof(T) == 4 && KC <= 8) {
+        launch_block_w<T, KC, 4>(SC, a, s, st);
+    } else if constexpr (sizeof(T) == 4 && KC <= 16) {
+        if (a.B > 512) launch_block_w<T, KC, 4>(SC, a, s, st);
+        else launch_block_w<T, KC, 1>(SC, a, s, st);
+    } else {
+        launch_block_w<T, KC, 1>(SC, a, s, st);
+    }
 }
 
 template <class T>
