@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/bnm_hip.h"
+#include "pool.hpp"
 
 namespace {
 
@@ -172,17 +173,19 @@ __global__ void k_fill_f32(float* __restrict__ p, int n, float v) {
 }
 
 // Adam (Kingma & Ba 2015) with bias correction
+__device__ __forceinline__ void adam_step(float* p, float* m1, float* m2, long i, float gi, float lr, float b1,
+                                          float b2, float eps, float c1, float c2) {
+    const float a = b1 * m1[i] + (1 - b1) * gi;
+    const float b = b2 * m2[i] + (1 - b2) * gi * gi;
+    m1[i] = a;
+    m2[i] = b;
+    p[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+}
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m1,
                        float* __restrict__ m2, long n, float lr, float b1, float b2, float eps,
                        float c1, float c2) {
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const float gi = g[i];
-        const float a = b1 * m1[i] + (1 - b1) * gi;
-        const float b = b2 * m2[i] + (1 - b2) * gi * gi;
-        m1[i] = a;
-        m2[i] = b;
-        p[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
-    }
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
+        adam_step(p, m1, m2, i, g[i], lr, b1, b2, eps, c1, c2);
 }
 
 // gather rows idx[0..n) of X [*, d] into out [n, d]
@@ -193,8 +196,11 @@ __global__ void k_gather(const float* __restrict__ X, const int* __restrict__ id
 }
 
 thread_local std::string g_mlp_err;
+constexpr int kLossBlocks = 64;
 
 }  // namespace
+
+#include "mlp_fused.hpp"
 
 struct bnm_mlp {
     int in = 0, hid = 0, depth = 0, out = 0, bf16 = 1;
@@ -211,6 +217,14 @@ struct bnm_mlp {
     int n_data = 0;
     long step = 0;
     hipStream_t st = nullptr;
+    // networks of layers up to 256 wide (mlp_fused.hpp): layer pointers, the
+    // weights' operand copies, and the buffers of a gradient for fcap rows
+    bool fused = false;
+    FusedNet net{};
+    FusedLayer layer[kFusedLayers];       // net.l is their copy on the device
+    void *wcopy = nullptr, *fbuf = nullptr;
+    int fcap = 0, xcap = 0, loss_cap = 0, idx_cap = 0, data_cap = 0;
+    float* px = nullptr;   // rows of a prediction or a loss_grad
 };
 
 namespace {
@@ -258,6 +272,115 @@ void gemm(bnm_mlp* m, const float* A, long sam, long sak, const float* B, long s
                        cz, M, N, K, klen, bias, Zout, Zin);
 }
 
+constexpr int kChunk = 65536;   // rows of a prediction at a time
+
+// ---- layers up to 256 wide -----------------------------------------------------
+size_t padded(int n, int to) { return (size_t)((n + to - 1) / to * to); }
+
+hipError_t put_layers(bnm_mlp* m) {
+    return hipMemcpy(const_cast<FusedLayer*>(m->net.l), m->layer, m->net.L * sizeof(FusedLayer), hipMemcpyHostToDevice);
+}
+
+// Gradient buffers for `rows` rows: gelu'(Z), dZ, the operands and the
+// weight gradients of the row splits.
+int ensure_fused(bnm_mlp* m, int rows) {
+    if (rows <= m->fcap) return BNM_OK;
+    if (m->fbuf) (void)hipFree(m->fbuf);
+    m->fbuf = nullptr;
+    m->fcap = 0;
+    const size_t es = m->bf16 ? 2 : 4, ldr = padded(rows, 32), kz = std::max(1, std::min(64, rows / 256));
+    size_t off = 0;
+    auto take = [&](size_t bytes) { const size_t o = off; off += (bytes + 255) / 256 * 256; return o; };
+    size_t o[kFusedLayers][5];
+    for (int l = 0; l < m->net.L; ++l) {
+        const size_t K = m->dims[l], N = m->dims[l + 1];
+        o[l][0] = take(ldr / 8 * kRowThreads * 4 * 4);
+        o[l][1] = take(ldr * N * 4);
+        o[l][2] = take(padded(K, 16) * ldr * es);
+        o[l][3] = take(padded(N, 16) * ldr * es);
+        o[l][4] = take(kz * N * K * 4);
+    }
+    MCHK(hipMalloc(&m->fbuf, off));
+    char* b = static_cast<char*>(m->fbuf);
+    for (int l = 0; l < m->net.L; ++l) {
+        FusedLayer& y = m->layer[l];
+        y.G = reinterpret_cast<float*>(b + o[l][0]);
+        y.dZ = reinterpret_cast<float*>(b + o[l][1]);
+        y.AT = b + o[l][2];
+        y.dT = b + o[l][3];
+        y.part = reinterpret_cast<float*>(b + o[l][4]);
+    }
+    MCHK(put_layers(m));
+    m->fcap = rows;
+    return BNM_OK;
+}
+
+int ensure_floats(float** p, int* cap, int n, size_t each) {
+    if (n <= *cap) return BNM_OK;
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+    *cap = 0;
+    MCHK(hipMalloc(p, (size_t)n * each * sizeof(float)));
+    *cap = n;
+    return BNM_OK;
+}
+
+// Rows per workgroup: eight while that gives no more than one workgroup a CU (a
+// step's latency counts); from two workgroups of 16 a CU on 32, so that the
+// weights are read half as often from L2 (not with FP32 operands: LDS).
+int block_rows(const bnm_mlp* m, int rows) { return rows <= 2048 ? 8 : m->bf16 && rows > 8192 ? 32 : 16; }
+
+template <bool BF16, bool TRAIN>
+void launch_rows(bnm_mlp* m, const FusedNet& n, int grid_rows) {
+    const int R = block_rows(m, n.rows);
+    const size_t smem = 2 * (size_t)R * (kFusedDim + Op<BF16>::EPV) * sizeof(typename Op<BF16>::E);
+    const dim3 grid((grid_rows + R - 1) / R);
+    if (R == 8) hipLaunchKernelGGL((k_mlp<BF16, 8, TRAIN>), grid, dim3(kRowThreads), smem, m->st, n);
+    else if (R == 16) hipLaunchKernelGGL((k_mlp<BF16, 16, TRAIN>), grid, dim3(kRowThreads), smem, m->st, n);
+    else hipLaunchKernelGGL((k_mlp<BF16, BF16 ? 32 : 16, TRAIN>), grid, dim3(kRowThreads), smem, m->st, n);
+}
+
+int fin(bnm_mlp* m, const FusedNet& n, int mode, float lr = 0, float b1 = 0, float b2 = 0, float eps = 0, float c1 = 1,
+        float c2 = 1) {
+    int most = 0;
+    for (int l = 0; l < n.L; ++l) most = std::max(most, steps_of(m->layer[l].N * (m->layer[l].K + 1), 256));
+    const dim3 grid(most, n.L);
+    if (m->bf16) hipLaunchKernelGGL(k_mlp_fin<true>, grid, dim3(256), 0, m->st, n, mode, m->p, m->g, m->m1, m->m2, lr, b1, b2, eps, c1, c2);
+    else hipLaunchKernelGGL(k_mlp_fin<false>, grid, dim3(256), 0, m->st, n, mode, m->p, m->g, m->m1, m->m2, lr, b1, b2, eps, c1, c2);
+    MCHK(hipGetLastError());
+    return BNM_OK;
+}
+
+// Partial sums of the loss that a gradient over `rows` rows leaves.
+int loss_parts(const bnm_mlp* m, int rows) {
+    const int R = block_rows(m, rows);
+    return (int)((padded(rows, 32) + R - 1) / R);
+}
+
+// forward and back over the rows of n, and the gradient's parts
+int fused_grad(bnm_mlp* m, FusedNet n) {
+    n.ldr = (int)padded(n.rows, 32);
+    n.scale = 1.0f / (float)((long)n.rows * m->out);
+    const int ks = std::max(1, std::min(64, n.rows / 256));
+    n.klen = (int)padded((n.rows + ks - 1) / ks, BK);
+    n.kz = (n.rows + n.klen - 1) / n.klen;
+    n.loss = m->loss_part;
+    // (rows up to ldr are written too, as zeros)
+    if (m->bf16) launch_rows<true, true>(m, n, n.ldr);
+    else launch_rows<false, true>(m, n, n.ldr);
+    int most = 0;
+    for (int l = 0; l < n.L; ++l) {
+        const FusedLayer& y = m->layer[l];
+        most = std::max(most, dw_tiles(y.N, y.K, n.kz) + steps_of(y.N, kColBlock));
+    }
+    const dim3 grid(most, n.L);
+    if (m->bf16) hipLaunchKernelGGL(k_mlp_dw<true>, grid, dim3(256), 0, m->st, n, m->g);
+    else hipLaunchKernelGGL(k_mlp_dw<false>, grid, dim3(256), 0, m->st, n, m->g);
+    m->net.kz = n.kz;
+    MCHK(hipGetLastError());
+    return BNM_OK;
+}
+
 // forward over `rows` rows already in A[0]; output in A[L]
 int forward(bnm_mlp* m, int rows) {
     const int L = m->depth + 1;
@@ -277,8 +400,6 @@ int forward(bnm_mlp* m, int rows) {
     MCHK(hipGetLastError());
     return BNM_OK;
 }
-
-constexpr int kLossBlocks = 64;
 
 // gradient into m->g for `rows` rows with targets in m->target; the loss goes
 // to m->loss_part (kLossBlocks partial sums, added to what is there when
@@ -350,6 +471,7 @@ bnm_mlp* bnm_mlp_create(int in_dim, int hidden, int depth, int out_dim, int bf16
         return nullptr;
     }
     auto* m = new bnm_mlp;
+    m->loss_cap = kLossBlocks;
     m->in = in_dim; m->hid = hidden; m->depth = depth; m->out = out_dim; m->bf16 = bf16 != 0;
     m->dims.push_back(in_dim);
     for (int i = 0; i < depth; ++i) m->dims.push_back(hidden);
@@ -375,7 +497,7 @@ bnm_mlp* bnm_mlp_create(int in_dim, int hidden, int depth, int out_dim, int bf16
               hipMalloc(&m->g, off * sizeof(float)) == hipSuccess &&
               hipMalloc(&m->m1, off * sizeof(float)) == hipSuccess &&
               hipMalloc(&m->m2, off * sizeof(float)) == hipSuccess &&
-              hipMalloc(&m->loss_part, 64 * sizeof(float)) == hipSuccess &&
+              hipMalloc(&m->loss_part, kLossBlocks * sizeof(float)) == hipSuccess &&
               hipMemcpy(m->p, h.data(), off * sizeof(float), hipMemcpyHostToDevice) == hipSuccess &&
               hipMemset(m->m1, 0, off * sizeof(float)) == hipSuccess &&
               hipMemset(m->m2, 0, off * sizeof(float)) == hipSuccess;
@@ -384,6 +506,42 @@ bnm_mlp* bnm_mlp_create(int in_dim, int hidden, int depth, int out_dim, int bf16
         set(BNM_E_HIP);
         bnm_mlp_destroy(m);
         return nullptr;
+    }
+    m->fused = depth + 1 <= kFusedLayers && std::max({in_dim, hidden, out_dim}) <= kFusedDim;
+    if (m->fused) {
+        const size_t es = m->bf16 ? 2 : 4;
+        const int ks = m->bf16 ? 32 : 16;
+        m->net.L = depth + 1;
+        size_t off = 0, of[kFusedLayers], ob[kFusedLayers];
+        for (int l = 0; l <= depth; ++l) {
+            const int K = m->dims[l], N = m->dims[l + 1];
+            of[l] = off;
+            off += padded(N, 16) * padded(K, ks) * es;
+            ob[l] = off;
+            off += padded(K, 16) * padded(N, ks) * es;
+        }
+        off = (off + 255) / 256 * 256;
+        ok = hipMalloc(&m->wcopy, off + sizeof(m->layer)) == hipSuccess && hipMemset(m->wcopy, 0, off) == hipSuccess &&
+             hipDeviceSynchronize() == hipSuccess;
+        m->net.W = static_cast<const unsigned*>(m->wcopy);
+        m->net.wwords = (unsigned)(off / 4);
+        m->net.l = reinterpret_cast<FusedLayer*>(static_cast<char*>(m->wcopy) + off);
+        for (int l = 0; l <= depth && ok; ++l) {
+            FusedLayer& y = m->layer[l] = FusedLayer{};
+            y.K = m->dims[l];
+            y.N = m->dims[l + 1];
+            y.Wf = static_cast<char*>(m->wcopy) + of[l];
+            y.Wb = static_cast<char*>(m->wcopy) + ob[l];
+            y.b = m->p + m->boff[l];
+            y.woff = (int)m->woff[l];
+            y.boff = (int)m->boff[l];
+        }
+        if (!ok || put_layers(m) != hipSuccess || fin(m, m->net, 0) != BNM_OK) {
+            g_mlp_err = "MLP allocation failed";
+            set(BNM_E_HIP);
+            bnm_mlp_destroy(m);
+            return nullptr;
+        }
     }
     set(BNM_OK);
     return m;
@@ -394,6 +552,8 @@ void bnm_mlp_destroy(bnm_mlp* m) {
     for (float* q : {m->p, m->g, m->m1, m->m2, m->part, m->loss_part, m->target, m->X, m->Y, m->bx, m->by})
         if (q) (void)hipFree(q);
     if (m->idx) (void)hipFree(m->idx);
+    for (void* q : {m->wcopy, m->fbuf, (void*)m->px})
+        if (q) (void)hipFree(q);
     for (auto* v : {&m->Z, &m->A, &m->dZ})
         for (float* q : *v)
             if (q) (void)hipFree(q);
@@ -414,13 +574,30 @@ int bnm_mlp_set_params(bnm_mlp* m, const float* in) {
     if (!m || !in) return BNM_E_ARG;
     MCHK(hipStreamSynchronize(m->st));
     MCHK(hipMemcpy(m->p, in, m->nparam * sizeof(float), hipMemcpyHostToDevice));
-    return BNM_OK;
+    return m->fused ? fin(m, m->net, 0) : BNM_OK;
 }
 
 // Y[n x out] = f(X[n x in])
 int bnm_mlp_predict(bnm_mlp* m, const float* X, int n, float* Y) {
     if (!m || !X || !Y || n < 1) return BNM_E_ARG;
-    const int chunk = 65536;
+    const int chunk = kChunk;
+    if (m->fused) {
+        int e = ensure_floats(&m->px, &m->xcap, std::min(n, chunk), m->in + m->out);
+        if (e) return e;
+        FusedNet f = m->net;
+        f.X = m->px;
+        f.Y = m->px + (size_t)m->xcap * m->in;
+        for (int s = 0; s < n; s += chunk) {
+            f.rows = std::min(chunk, n - s);
+            MCHK(hipMemcpyAsync(m->px, X + (long)s * m->in, (size_t)f.rows * m->in * sizeof(float), hipMemcpyHostToDevice, m->st));
+            if (m->bf16) launch_rows<true, false>(m, f, f.rows);
+            else launch_rows<false, false>(m, f, f.rows);
+            MCHK(hipGetLastError());
+            MCHK(hipMemcpyAsync(Y + (long)s * m->out, f.Y, (size_t)f.rows * m->out * sizeof(float), hipMemcpyDeviceToHost, m->st));
+            MCHK(hipStreamSynchronize(m->st));
+        }
+        return BNM_OK;
+    }
     for (int s = 0; s < n; s += chunk) {
         const int r = std::min(chunk, n - s);
         int e = ensure_rows(m, r);
@@ -438,8 +615,32 @@ int bnm_mlp_predict(bnm_mlp* m, const float* X, int n, float* Y) {
 // parameter vector at the current parameters.
 int bnm_mlp_loss_grad(bnm_mlp* m, const float* X, const float* T, int n, float* loss, float* grad) {
     if (!m || !X || !T || n < 1) return BNM_E_ARG;
-    int e = ensure_rows(m, n);
-    if (e) return e;
+    int e = 0;
+    if (m->fused) {
+        const int parts = loss_parts(m, n);
+        if ((e = ensure_fused(m, n))) return e;
+        if ((e = ensure_floats(&m->px, &m->xcap, n, m->in + m->out))) return e;
+        if ((e = ensure_floats(&m->loss_part, &m->loss_cap, parts, 1))) return e;
+        FusedNet f = m->net;
+        f.rows = n;
+        f.X = m->px;
+        f.T = m->px + (size_t)m->xcap * m->in;
+        MCHK(hipMemcpyAsync(m->px, X, (size_t)n * m->in * sizeof(float), hipMemcpyHostToDevice, m->st));
+        MCHK(hipMemcpyAsync(const_cast<float*>(f.T), T, (size_t)n * m->out * sizeof(float), hipMemcpyHostToDevice, m->st));
+        if ((e = fused_grad(m, f))) return e;
+        if ((e = fin(m, m->net, 1))) return e;
+        std::vector<float> lp(parts);
+        MCHK(hipMemcpyAsync(lp.data(), m->loss_part, parts * sizeof(float), hipMemcpyDeviceToHost, m->st));
+        if (grad) MCHK(hipMemcpyAsync(grad, m->g, m->nparam * sizeof(float), hipMemcpyDeviceToHost, m->st));
+        MCHK(hipStreamSynchronize(m->st));
+        if (loss) {
+            double s = 0;
+            for (float v : lp) s += v;
+            *loss = (float)s;
+        }
+        return BNM_OK;
+    }
+    if ((e = ensure_rows(m, n))) return e;
     MCHK(hipMemcpyAsync(m->A[0], X, (size_t)n * m->in * sizeof(float), hipMemcpyHostToDevice, m->st));
     MCHK(hipMemcpyAsync(m->target, T, (size_t)n * m->out * sizeof(float), hipMemcpyHostToDevice, m->st));
     if ((e = forward(m, n))) return e;
@@ -453,10 +654,14 @@ int bnm_mlp_loss_grad(bnm_mlp* m, const float* X, const float* T, int n, float* 
 int bnm_mlp_set_data(bnm_mlp* m, const float* X, const float* T, int n) {
     if (!m || !X || !T || n < 1) return BNM_E_ARG;
     MCHK(hipStreamSynchronize(m->st));
-    for (float** q : {&m->X, &m->Y})
-        if (*q) { (void)hipFree(*q); *q = nullptr; }
-    MCHK(hipMalloc(&m->X, (size_t)n * m->in * sizeof(float)));
-    MCHK(hipMalloc(&m->Y, (size_t)n * m->out * sizeof(float)));
+    if (n > m->data_cap) {   // (a set that fits goes where the last one was)
+        for (float** q : {&m->X, &m->Y})
+            if (*q) { (void)hipFree(*q); *q = nullptr; }
+        m->n_data = m->data_cap = 0;
+        MCHK(hipMalloc(&m->X, (size_t)n * m->in * sizeof(float)));
+        MCHK(hipMalloc(&m->Y, (size_t)n * m->out * sizeof(float)));
+        m->data_cap = n;
+    }
     MCHK(hipMemcpy(m->X, X, (size_t)n * m->in * sizeof(float), hipMemcpyHostToDevice));
     MCHK(hipMemcpy(m->Y, T, (size_t)n * m->out * sizeof(float), hipMemcpyHostToDevice));
     m->n_data = n;
@@ -468,24 +673,43 @@ int bnm_mlp_set_data(bnm_mlp* m, const float* X, const float* T, int n) {
 int bnm_mlp_train(bnm_mlp* m, int epochs, int batch, float lr, unsigned seed, float* loss) {
     if (!m || m->n_data < 1 || batch < 1 || epochs < 1) return BNM_E_ARG;
     batch = std::min(batch, m->n_data);
-    int e = ensure_rows(m, batch);
+    int e = m->fused ? ensure_fused(m, batch) : ensure_rows(m, batch);
     if (e) return e;
-    if (m->idx) { (void)hipFree(m->idx); m->idx = nullptr; }
-    MCHK(hipMalloc(&m->idx, (size_t)m->n_data * sizeof(int)));
+    const int parts = m->fused ? loss_parts(m, batch) : kLossBlocks;
+    if ((e = ensure_floats(&m->loss_part, &m->loss_cap, parts, 1))) return e;
+    if (m->idx_cap < m->n_data) {
+        if (m->idx) { (void)hipFree(m->idx); m->idx = nullptr; }
+        m->idx_cap = 0;
+        MCHK(hipMalloc(&m->idx, (size_t)m->n_data * sizeof(int)));
+        m->idx_cap = m->n_data;
+    }
     std::mt19937 gen(seed);
     std::vector<int> perm(m->n_data);
     for (int i = 0; i < m->n_data; ++i) perm[i] = i;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const int nb = m->n_data / batch;
-    float lp[kLossBlocks];
+    std::vector<float> lp(parts);
     for (int ep = 0; ep < epochs; ++ep) {
         std::shuffle(perm.begin(), perm.end(), gen);
         // the previous epoch's kernels read m->idx: the synchronous copy waits for them
         MCHK(hipStreamSynchronize(m->st));
         MCHK(hipMemcpy(m->idx, perm.data(), (size_t)m->n_data * sizeof(int), hipMemcpyHostToDevice));
-        hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(64), 0, m->st, m->loss_part, kLossBlocks, 0.0f);
+        hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(64), 0, m->st, m->loss_part, parts, 0.0f);
         for (int b = 0; b < nb; ++b) {
             const int* ib = m->idx + (long)b * batch;
+            if (m->fused) {
+                FusedNet f = m->net;
+                f.rows = batch;
+                f.X = m->X;
+                f.T = m->Y;
+                f.idx = ib;
+                f.accum = 1;
+                if ((e = fused_grad(m, f))) return e;
+                ++m->step;
+                const float c1 = 1 - std::pow(b1, (float)m->step), c2 = 1 - std::pow(b2, (float)m->step);
+                if ((e = fin(m, m->net, 2, lr, b1, b2, eps, c1, c2))) return e;
+                continue;
+            }
             hipLaunchKernelGGL(k_gather, dim3(256), dim3(256), 0, m->st, m->X, ib, batch, m->in, m->A[0]);
             hipLaunchKernelGGL(k_gather, dim3(256), dim3(256), 0, m->st, m->Y, ib, batch, m->out, m->target);
             if ((e = forward(m, batch))) return e;
@@ -497,7 +721,7 @@ int bnm_mlp_train(bnm_mlp* m, int epochs, int batch, float lr, unsigned seed, fl
         }
         MCHK(hipGetLastError());
         if (loss) {
-            MCHK(hipMemcpyAsync(lp, m->loss_part, sizeof(lp), hipMemcpyDeviceToHost, m->st));
+            MCHK(hipMemcpyAsync(lp.data(), m->loss_part, parts * sizeof(float), hipMemcpyDeviceToHost, m->st));
             MCHK(hipStreamSynchronize(m->st));
             double ls = 0;
             for (float v : lp) ls += v;
