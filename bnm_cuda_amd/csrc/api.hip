@@ -89,6 +89,7 @@ struct bnm_ctx {
     bool fcsplit = false; // ... as hi/lo pairs (three products)
     bool fcd_direct = false;
     int fcd_tile = 64;
+    int win_len = 0;      // longest FCD window
     bool have_bold = false;  // BOLD holds a run's or a caller's series
     hipStream_t st = nullptr;
     double* SC64 = nullptr;
@@ -434,6 +435,7 @@ static int ctx_alloc(bnm_ctx* x) {
         for (int w = 0; w + 1 < x->nseg; ++w) {
             st[w + 1] = ws[w];
             ln[w + 1] = we[w] - ws[w] + 1;
+            x->win_len = std::max(x->win_len, ln[w + 1]);
         }
         if ((r = cdalloc(x, &x->seg_start, x->nseg))) return r;
         if ((r = cdalloc(x, &x->seg_len, x->nseg))) return r;
@@ -1126,7 +1128,7 @@ static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only
             if (x->fc64)
                 HIPCHK((launch_gram_fc<double, double, double>(
                     (const double*)x->bold, x->B, x->N, x->ots, x->nseg, x->seg_start, x->seg_len,
-                    x->mean, x->inv, x->pidx, x->np, (double*)x->fc, (double*)x->wfc, st)));
+                    x->mean, x->inv, x->pidx, x->np, (double*)x->fc, (double*)x->wfc, st, x->win_len, x->lds_max)));
             else if (x->fcbf16)
                 HIPCHK(launch_gram_fc_bf16<double>(
                     (const double*)x->bold, x->B, x->N, x->ots, x->nseg, x->seg_start, x->seg_len,
@@ -1134,14 +1136,14 @@ static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only
             else
                 HIPCHK((launch_gram_fc<double, float, float>(
                     (const double*)x->bold, x->B, x->N, x->ots, x->nseg, x->seg_start, x->seg_len,
-                    x->mean, x->inv, x->pidx, x->np, (float*)x->fc, (float*)x->wfc, st)));
+                    x->mean, x->inv, x->pidx, x->np, (float*)x->fc, (float*)x->wfc, st, x->win_len, x->lds_max)));
         } else {
             HIPCHK(launch_seg_moments<float>((const float*)x->bold, x->B, x->N, x->ots, x->nseg,
                                              x->seg_start, x->seg_len, x->mean, x->inv, st));
             if (x->fc64)
                 HIPCHK((launch_gram_fc<float, double, double>(
                     (const float*)x->bold, x->B, x->N, x->ots, x->nseg, x->seg_start, x->seg_len,
-                    x->mean, x->inv, x->pidx, x->np, (double*)x->fc, (double*)x->wfc, st)));
+                    x->mean, x->inv, x->pidx, x->np, (double*)x->fc, (double*)x->wfc, st, x->win_len, x->lds_max)));
             else if (x->fcbf16)
                 HIPCHK(launch_gram_fc_bf16<float>(
                     (const float*)x->bold, x->B, x->N, x->ots, x->nseg, x->seg_start, x->seg_len,
@@ -1149,7 +1151,7 @@ static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only
             else
                 HIPCHK((launch_gram_fc<float, float, float>(
                     (const float*)x->bold, x->B, x->N, x->ots, x->nseg, x->seg_start, x->seg_len,
-                    x->mean, x->inv, x->pidx, x->np, (float*)x->fc, (float*)x->wfc, st)));
+                    x->mean, x->inv, x->pidx, x->np, (float*)x->fc, (float*)x->wfc, st, x->win_len, x->lds_max)));
         }
     }
     if (timed) HIPCHK(hipEventRecord(x->ev[3], st));

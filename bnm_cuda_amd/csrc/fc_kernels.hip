@@ -6,6 +6,8 @@
 // ssd_i = sqrt(sum_t (x_ti - mean_i)^2).  The moments are FP64 sums with
 // Neumaier compensation; the cross products run on MFMA in the Gram precision
 // (FP64: v_mfma_f64_16x16x4f64, FP32: v_mfma_f32_16x16x4f32).
+#include <type_traits>
+
 #include "kernels.hpp"
 
 namespace bnm {
@@ -41,6 +43,9 @@ __device__ double block_sum(double v, double* red) {
 }  // namespace
 
 // ---- node moments per (sim, segment) -----------------------------------------
+// A thread per (segment, node).  Bound by latency (a compensated sum is a chain,
+// and its loads waited for it one by one): eight loads at a time.  16 sims x 1158
+// segments of 45 x 400 nodes: 1.4 ms -> 0.44.
 template <class T>
 __global__ __launch_bounds__(256) void k_seg_moments(const T* __restrict__ bold, int N,
                                                      int output_ts, int n_seg,
@@ -48,22 +53,35 @@ __global__ __launch_bounds__(256) void k_seg_moments(const T* __restrict__ bold,
                                                      const int* __restrict__ seg_len,
                                                      double* __restrict__ mean,
                                                      double* __restrict__ inv_ssd) {
-    const int seg = blockIdx.x, sim = blockIdx.y;
-    const int t0 = seg_start[seg], len = seg_len[seg];
-    const T* x = bold + ((size_t)sim * output_ts + t0) * N;
-    for (int j = threadIdx.x; j < N; j += blockDim.x) {
-        KSum s;
-        for (int t = 0; t < len; ++t) s.add(to_d(x[(size_t)t * N + j]));
-        const double m = s.value() / len;
-        KSum q;
-        for (int t = 0; t < len; ++t) {
-            const double d = to_d(x[(size_t)t * N + j]) - m;
-            q.add(d * d);
+    const long long i = blockIdx.x * 256LL + threadIdx.x;
+    const int sim = blockIdx.y;
+    if (i >= (long long)n_seg * N) return;
+    const int seg = (int)(i / N), j = (int)(i % N);
+    const int len = seg_len[seg];
+    const T* x = bold + ((size_t)sim * output_ts + seg_start[seg]) * N + j;
+    constexpr int U = 8;
+    auto each = [&](auto f) {
+        int t = 0;
+        for (; t + U <= len; t += U) {
+            T v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = x[(size_t)(t + u) * N];
+#pragma unroll
+            for (int u = 0; u < U; ++u) f(to_d(v[u]));
         }
-        const size_t o = ((size_t)sim * n_seg + seg) * N + j;
-        mean[o] = m;
-        inv_ssd[o] = 1.0 / sqrt(q.value());
-    }
+        for (; t < len; ++t) f(to_d(x[(size_t)t * N]));
+    };
+    KSum s;
+    each([&](double v) { s.add(v); });
+    const double m = s.value() / len;
+    KSum q;
+    each([&](double v) {
+        const double d = v - m;
+        q.add(d * d);
+    });
+    const size_t o = (size_t)sim * n_seg * N + i;
+    mean[o] = m;
+    inv_ssd[o] = 1.0 / sqrt(q.value());
 }
 
 // ---- row moments (window-FC rows over the edge axis) -------------------------
@@ -145,26 +163,39 @@ __device__ void gram_tile(const GramItem& it, int ti, int tj, const int* __restr
     V4 acc[2][2];
     for (int a = 0; a < 2; ++a)
         for (int b = 0; b < 2; ++b) acc[a][b] = V4{0, 0, 0, 0};
+    // loader: RL values of each operand a thread, the next chunk's in flight behind
+    // this one's products
+    constexpr int RL = TK * TM / 256;
     const bool mfast = it.ldm == 1;
+    Tin xa[RL], xb[RL];
+    double mua[RL], isa[RL], mub[RL], isb[RL];
+    const auto m_of = [&](int r) { const int e = tid + 256 * r; return mfast ? e % TM : e / TK; };
+    const auto k_of = [&](int r) { const int e = tid + 256 * r; return mfast ? e / TM : e % TK; };
+#pragma unroll
+    for (int r = 0; r < RL; ++r) {
+        const int mi = min(ti * TM + m_of(r), it.M - 1), mj = min(tj * TM + m_of(r), it.M - 1);
+        mua[r] = it.mu[mi]; isa[r] = it.is[mi];
+        mub[r] = it.mu[mj]; isb[r] = it.is[mj];
+    }
+    const auto load = [&](int k0) {   // (rows and columns past the last repeat it and are not used)
+#pragma unroll
+        for (int r = 0; r < RL; ++r) {
+            const size_t kg = (size_t)min(k0 + k_of(r), it.K - 1) * it.ldk;
+            xa[r] = X[kg + (size_t)min(ti * TM + m_of(r), it.M - 1) * it.ldm];
+            xb[r] = X[kg + (size_t)min(tj * TM + m_of(r), it.M - 1) * it.ldm];
+        }
+    };
+    load(0);
     for (int k0 = 0; k0 < it.K; k0 += TK) {
 #pragma unroll
-        for (int r = 0; r < (TK * TM) / 256; ++r) {
-            const int e = tid + 256 * r;
-            const int m = mfast ? (e % TM) : (e / TK);
-            const int k = mfast ? (e / TM) : (e % TK);
-            const int kg = k0 + k;
-            const int mi = ti * TM + m, mj = tj * TM + m;
-            Tc za = 0, zb = 0;
-            if (kg < it.K) {
-                if (mi < it.M)
-                    za = (Tc)((to_d(X[(size_t)kg * it.ldk + (size_t)mi * it.ldm]) - it.mu[mi]) * it.is[mi]);
-                if (mj < it.M)
-                    zb = (Tc)((to_d(X[(size_t)kg * it.ldk + (size_t)mj * it.ldm]) - it.mu[mj]) * it.is[mj]);
-            }
-            As[k][m] = za;
-            Bs[k][m] = zb;
+        for (int r = 0; r < RL; ++r) {
+            const int m = m_of(r), k = k_of(r);
+            const bool in = k0 + k < it.K;
+            As[k][m] = in && ti * TM + m < it.M ? (Tc)((to_d(xa[r]) - mua[r]) * isa[r]) : (Tc)0;
+            Bs[k][m] = in && tj * TM + m < it.M ? (Tc)((to_d(xb[r]) - mub[r]) * isb[r]) : (Tc)0;
         }
         __syncthreads();
+        if (k0 + TK < it.K) load(k0 + TK);
 #pragma unroll
         for (int kk = 0; kk < TK / 4; ++kk) {
             const int kr = kk * 4 + (lane >> 4);
@@ -358,6 +389,120 @@ __global__ __launch_bounds__(256) void k_gram_fc(const Tin* __restrict__ bold, i
     it.out = seg == 0 ? (void*)(fc + (size_t)sim * np)
                       : (void*)(wfc + ((size_t)sim * (n_seg - 1) + (seg - 1)) * np);
     gram_tile<Tin, Tc, Tout>(it, ti, tj, pidx, As, Bs);
+}
+
+// The windows (segments from 1 on) of a simulation, one workgroup each: the
+// window is z-scored once into LDS, [k][node], and all its 32 x 32 output tiles
+// are formed from there, a wave a tile; tiles with no pair in the list are left
+// out.  The 64 x 64 tiles of k_gram_fc z-score each value again for every tile of
+// its row and column (FP64: 7 of 10 cycles at N = 400), and wait for their loads
+// before every 16 steps of k.  Same products in the same order of k, so the same
+// bits.  Bound by the matrix pipes and the writes: 16 sims x 1157 windows of 45 x
+// 400 nodes, FP32, pairs of the same hemisphere: 5.0 ms -> 2.0 (the writes alone
+// take 0.6, the products 0.6).
+// Row stride: 16 banks further each step of k, so that the four steps of a
+// fragment's lanes lie in different banks.
+__host__ __device__ constexpr int win_stride(int N, int elem) {
+    const int per = elem == 8 ? 32 : 64;
+    return (N + per - 17) / per * per + 16;
+}
+
+template <class Tin, class Tc, class Tout>
+__global__ __launch_bounds__(512) void k_gram_win(const Tin* __restrict__ bold, int N, int output_ts, int n_seg,
+                                                  const int* __restrict__ seg_start, const int* __restrict__ seg_len,
+                                                  const double* __restrict__ mean, const double* __restrict__ inv_ssd,
+                                                  const int* __restrict__ pidx, int np, Tout* __restrict__ wfc) {
+    using V4 = typename MF<Tc>::v4;
+    extern __shared__ __align__(16) unsigned char zmem[];
+    Tc* Z = reinterpret_cast<Tc*>(zmem);
+    const int S = win_stride(N, sizeof(Tc));
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, waves = blockDim.x >> 6;
+    const int seg = blockIdx.x + 1, sim = blockIdx.y;
+    const int len = seg_len[seg], kp = (len + 3) & ~3;
+    const Tin* x = bold + ((size_t)sim * output_ts + seg_start[seg]) * N;
+    const double* mu = mean + ((size_t)sim * n_seg + seg) * N;
+    const double* is = inv_ssd + ((size_t)sim * n_seg + seg) * N;
+    {
+        int k = tid / N, m = tid % N;
+        const int dk = blockDim.x / N, dm = blockDim.x % N;
+        constexpr int U = 4;   // loads in flight
+        for (int e = tid; e < len * N; e += U * blockDim.x) {
+            Tin v[U];
+            double a[U], b[U];
+            int at[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                v[u] = x[min(e + u * (int)blockDim.x, len * N - 1)];
+                a[u] = mu[m];
+                b[u] = is[m];
+                at[u] = k * S + m;
+                k += dk;
+                m += dm;
+                if (m >= N) { m -= N; ++k; }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (e + u * (int)blockDim.x < len * N) Z[at[u]] = (Tc)((to_d(v[u]) - a[u]) * b[u]);
+        }
+        for (int e = tid; e < (kp - len) * N; e += blockDim.x) Z[(len + e / N) * S + e % N] = (Tc)0;
+    }
+    __syncthreads();
+    const int g = lane >> 4, c = lane & 15, nt = (N + 31) / 32;
+    Tout* out = wfc + ((size_t)sim * (n_seg - 1) + (seg - 1)) * np;
+    int ti = 0, tj = w;
+    for (;; tj += waves) {
+        while (tj > ti) tj -= ++ti;      // (rows hold 1, 2, 3, ... tiles)
+        if (ti >= nt) break;
+        int p[2][2][4];
+        int any = 0;
+#pragma unroll
+        for (int qa = 0; qa < 2; ++qa)
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = ti * 32 + qa * 16 + MF<Tc>::row(lane, r), col = tj * 32 + qb * 16 + c;
+                    p[qa][qb][r] = row < N && col < row ? pidx[(size_t)row * N + col] : -1;
+                    any |= p[qa][qb][r] >= 0;
+                }
+        if (!__any(any)) continue;
+        V4 acc[2][2];
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) acc[a][b] = V4{0, 0, 0, 0};
+        const Tc* A = Z + g * S + ti * 32 + c;
+        const Tc* B = Z + g * S + tj * 32 + c;
+        auto steps = [&](auto un) __attribute__((always_inline)) {
+            constexpr int U = decltype(un)::value;
+            Tc a[U][2], b[U][2];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    a[u][q] = A[4 * u * S + 16 * q];
+                    b[u][q] = B[4 * u * S + 16 * q];
+                }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int qa = 0; qa < 2; ++qa)
+#pragma unroll
+                    for (int qb = 0; qb < 2; ++qb) acc[qa][qb] = MF<Tc>::mma(a[u][qa], b[u][qb], acc[qa][qb]);
+            A += 4 * U * S;
+            B += 4 * U * S;
+        };
+        int k = 0;
+        for (; k + 16 <= kp; k += 16) steps(std::integral_constant<int, 4>{});
+        for (; k < kp; k += 4) steps(std::integral_constant<int, 1>{});
+#pragma unroll
+        for (int qa = 0; qa < 2; ++qa)
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (p[qa][qb][r] >= 0) out[p[qa][qb][r]] = (Tout)acc[qa][qb][r];
+    }
 }
 
 template <class Tin, class Tc, class Tout>
@@ -648,8 +793,7 @@ template <class T>
 hipError_t launch_seg_moments(const T* bold, int B, int N, int output_ts, int n_seg,
                               const int* seg_start, const int* seg_len, double* mean,
                               double* inv_ssd, hipStream_t st) {
-    const int threads = N >= 256 ? 256 : ((N + 63) / 64) * 64;
-    hipLaunchKernelGGL(k_seg_moments<T>, dim3(n_seg, B), dim3(threads), 0, st, bold, N, output_ts,
+    hipLaunchKernelGGL(k_seg_moments<T>, dim3((unsigned)(((long long)n_seg * N + 255) / 256), B), dim3(256), 0, st, bold, N, output_ts,
                        n_seg, seg_start, seg_len, mean, inv_ssd);
     return hipGetLastError();
 }
@@ -667,9 +811,21 @@ template <class Tin, class Tc, class Tout>
 hipError_t launch_gram_fc(const Tin* bold, int B, int N, int output_ts, int n_seg,
                           const int* seg_start, const int* seg_len, const double* mean,
                           const double* inv_ssd, const int* pidx, int np, Tout* fc, Tout* wfc,
-                          hipStream_t st) {
+                          hipStream_t st, int win_len, size_t lds_max) {
     const int nt = (N + TM - 1) / TM;
-    hipLaunchKernelGGL((k_gram_fc<Tin, Tc, Tout>), dim3(nt * (nt + 1) / 2, n_seg, B), dim3(256), 0,
+    // Windows that fit LDS go to k_gram_win whenever there are any (the whole
+    // series stays with k_gram_fc: one workgroup would have all its tiles).  k_gram_fc
+    // against it: 400 nodes x 45, FP32, 16 sims x 1157 windows, 5.0 and 2.0 ms; 100
+    // nodes x 31, FP64, 128 x 79, 0.69 and 0.17 ms.  With a few tiles, four waves
+    // share them evenly; with many, eight.
+    const size_t lds = ((size_t)((win_len + 3) & ~3) * win_stride(N, sizeof(Tc)) + 32) * sizeof(Tc);
+    const bool win = n_seg > 1 && lds <= lds_max;
+    if (win) {
+        const int n32 = (N + 31) / 32, tiles = n32 * (n32 + 1) / 2;
+        hipLaunchKernelGGL((k_gram_win<Tin, Tc, Tout>), dim3(n_seg - 1, B), dim3(tiles <= 16 ? 256 : 512), lds, st, bold,
+                           N, output_ts, n_seg, seg_start, seg_len, mean, inv_ssd, pidx, np, wfc);
+    }
+    hipLaunchKernelGGL((k_gram_fc<Tin, Tc, Tout>), dim3(nt * (nt + 1) / 2, win ? 1 : n_seg, B), dim3(256), 0,
                        st, bold, N, output_ts, n_seg, seg_start, seg_len, mean, inv_ssd, pidx, np,
                        fc, wfc);
     return hipGetLastError();
@@ -729,7 +885,7 @@ BNM_INST_MOM(double)
 #define BNM_INST_FC(Tin, Tc)                                                                      \
     template hipError_t launch_gram_fc<Tin, Tc, Tc>(const Tin*, int, int, int, int, const int*,   \
                                                     const int*, const double*, const double*,     \
-                                                    const int*, int, Tc*, Tc*, hipStream_t);
+                                                    const int*, int, Tc*, Tc*, hipStream_t, int, size_t);
 BNM_INST_FC(double, double)
 BNM_INST_FC(double, float)
 BNM_INST_FC(float, double)

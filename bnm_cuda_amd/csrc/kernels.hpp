@@ -152,7 +152,7 @@ template <class Tin, class Tc, class Tout>
 hipError_t launch_gram_fc(const Tin* bold, int B, int N, int output_ts, int n_seg,
                           const int* seg_start, const int* seg_len, const double* mean,
                           const double* inv_ssd, const int* pidx, int np, Tout* fc, Tout* wfc,
-                          hipStream_t st);
+                          hipStream_t st, int win_len, size_t lds_max);   // longest window; LDS a workgroup may use
 template <class Tin, class Tc, class Tout>
 hipError_t launch_gram_fcd(const Tin* wfc, int B, int nw, int np, const double* mean,
                            const double* inv_ssd, Tout* fcd, hipStream_t st, int col0 = 0, int K = -1);
