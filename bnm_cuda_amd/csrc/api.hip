@@ -1186,11 +1186,12 @@ static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only
             HIPCHK((launch_gram_fcd<double, double, double>((const double*)x->wfc, x->B, x->nw, x->np,
                                                             x->wmean, x->winv, (double*)x->fcd, st)));
         } else {
-            HIPCHK(launch_row_moments<float>((const float*)x->wfc, (long long)x->B * x->nw, x->np,
-                                             x->wmean, x->winv, st));
+            if (!x->wz)
+                HIPCHK(launch_row_moments<float>((const float*)x->wfc, (long long)x->B * x->nw, x->np,
+                                                 x->wmean, x->winv, st));
             if (x->wz)
-                HIPCHK(launch_fcd_z((const float*)x->wfc, x->B, x->nw, x->np, x->wmean, x->winv, x->wz, x->wzlo,
-                                    x->fcsplit ? 2 : x->fcbf16 ? 1 : 0, (float*)x->fcd, st, x->fcd_tile));
+                HIPCHK(launch_fcd_z((const float*)x->wfc, x->B, x->nw, x->np, x->wz, x->wzlo,
+                                    x->fcsplit ? 2 : x->fcbf16 ? 1 : 0, (float*)x->fcd, st, x->fcd_tile, x->lds_max));
             else if (x->fcbf16)
                 HIPCHK(launch_gram_fcd_bf16((const float*)x->wfc, x->B, x->nw, x->np, x->wmean, x->winv,
                                             (float*)x->fcd, x->fcsplit, st));

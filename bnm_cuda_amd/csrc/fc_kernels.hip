@@ -43,9 +43,12 @@ __device__ double block_sum(double v, double* red) {
 }  // namespace
 
 // ---- node moments per (sim, segment) -----------------------------------------
-// A thread per (segment, node).  Bound by latency (a compensated sum is a chain,
-// and its loads waited for it one by one): eight loads at a time.  16 sims x 1158
-// segments of 45 x 400 nodes: 1.4 ms -> 0.44.
+// A workgroup takes 64 (segment, node) columns, each of its four waves a quarter of
+// the segment.  Bound by latency (a compensated sum is a chain, and its loads were
+// waited for one by one; the whole series, the longest, is the last to end): four
+// loads at a time, quarters added in order.  16 sims x 1158 segments of 45 x 400
+// nodes, FP32: 1.4 ms -> 0.5; 128 x 80 of 31 x 100 with a series of 421, FP64:
+// 0.34 -> 0.08.
 template <class T>
 __global__ __launch_bounds__(256) void k_seg_moments(const T* __restrict__ bold, int N,
                                                      int output_ts, int n_seg,
@@ -53,35 +56,44 @@ __global__ __launch_bounds__(256) void k_seg_moments(const T* __restrict__ bold,
                                                      const int* __restrict__ seg_len,
                                                      double* __restrict__ mean,
                                                      double* __restrict__ inv_ssd) {
-    const long long i = blockIdx.x * 256LL + threadIdx.x;
-    const int sim = blockIdx.y;
-    if (i >= (long long)n_seg * N) return;
-    const int seg = (int)(i / N), j = (int)(i % N);
-    const int len = seg_len[seg];
+    constexpr int P = 4, U = 4;
+    __shared__ double part[2][P][2][64];
+    const int lane = threadIdx.x & 63, p = threadIdx.x >> 6, sim = blockIdx.y;
+    const long long cols = (long long)n_seg * N, i = blockIdx.x * 64LL + lane, ic = i < cols ? i : cols - 1;
+    const int seg = (int)(ic / N), j = (int)(ic % N);
+    const int len = seg_len[seg], q = (len + P - 1) / P, t0 = min(len, p * q), t1 = min(len, t0 + q);
     const T* x = bold + ((size_t)sim * output_ts + seg_start[seg]) * N + j;
-    constexpr int U = 8;
-    auto each = [&](auto f) {
-        int t = 0;
-        for (; t + U <= len; t += U) {
+    // sum of f(x) over the segment, for all quarters' threads
+    auto sum = [&](int pass, auto f) __attribute__((always_inline)) {
+        KSum s;
+        int t = t0;
+        for (; t + U <= t1; t += U) {
             T v[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) v[u] = x[(size_t)(t + u) * N];
 #pragma unroll
-            for (int u = 0; u < U; ++u) f(to_d(v[u]));
+            for (int u = 0; u < U; ++u) s.add(f(to_d(v[u])));
         }
-        for (; t < len; ++t) f(to_d(x[(size_t)t * N]));
+        for (; t < t1; ++t) s.add(f(to_d(x[(size_t)t * N])));
+        part[pass][p][0][lane] = s.s;
+        part[pass][p][1][lane] = s.c;
+        __syncthreads();
+        KSum all;
+        double c = 0;
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+            all.add(part[pass][r][0][lane]);
+            c += part[pass][r][1][lane];
+        }
+        return all.s + (all.c + c);
     };
-    KSum s;
-    each([&](double v) { s.add(v); });
-    const double m = s.value() / len;
-    KSum q;
-    each([&](double v) {
-        const double d = v - m;
-        q.add(d * d);
-    });
-    const size_t o = (size_t)sim * n_seg * N + i;
-    mean[o] = m;
-    inv_ssd[o] = 1.0 / sqrt(q.value());
+    const double m = sum(0, [](double v) { return v; }) / len;
+    const double ss = sum(1, [m](double v) { return (v - m) * (v - m); });
+    if (p == 0 && i < cols) {
+        const size_t o = (size_t)sim * cols + i;
+        mean[o] = m;
+        inv_ssd[o] = 1.0 / sqrt(ss);
+    }
 }
 
 // ---- row moments (window-FC rows over the edge axis) -------------------------
@@ -149,6 +161,15 @@ __device__ __forceinline__ void tile_pair(int p, int& ti, int& tj) {
     ti = t;
     tj = p - t * (t + 1) / 2;
 }
+
+// Work item of a workgroup: the `total` (simulation, tile) items in order, an
+// eighth to each XCD (workgroup i runs on XCD i mod 8), so that the tiles that run
+// together on an XCD share rows in its L2.  -1: none.
+__device__ __forceinline__ int xcd_item(unsigned block, int total) {
+    const int per = (total + 7) / 8, i = (int)(block >> 3) + (int)(block & 7) * per;
+    return (int)(block >> 3) < per && i < total ? i : -1;
+}
+inline unsigned xcd_grid(int total) { return 8u * ((total + 7) / 8); }
 
 // One 64x64 lower-triangle output tile (ti >= tj) of the Gram of item `it`.
 // pidx: pair index table [M*M] (-1 = not in the list) or nullptr for the
@@ -505,6 +526,97 @@ __global__ __launch_bounds__(512) void k_gram_win(const Tin* __restrict__ bold, 
     }
 }
 
+// FP64 FCD, rows z-scored on the way: an output tile of 32 x 32 a workgroup, each
+// wave a quarter of the edges, added up in order.  A lane reads four consecutive
+// edges of a row (which edges meet in one MFMA does not matter), the next 16 of its
+// rows on the way behind the products of these.  Tiles of one simulation run on one
+// XCD and share its rows in L2.  64 x 64 tiles staged through LDS, 16 edges at a
+// time, waited 3 us for 0.4 us of products: 128 sims x 79 rows of 2450, 0.58 ms (0.45
+// with the next chunk in flight) -> 0.115; four quadrants of 64 x 64 instead of four
+// quarters of the edges: 1.07 times as long with 3584 tiles, 1.5 times with 190.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gram_fcd64(
+    const double* __restrict__ wfc, int nw, int np, int col0, int K, const double* __restrict__ mean,
+    const double* __restrict__ inv_ssd, int tiles, int total, double* __restrict__ fcd) {
+    typedef MF<double>::v4 V4;
+    __shared__ double part[4 * 16 * 64];
+    constexpr int KC = 16, V = 4;
+    const int item = xcd_item(blockIdx.x, total);
+    if (item < 0) return;
+    const int sim = item / tiles, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
+    int ti, tj;
+    tile_pair(item % tiles, ti, tj);
+    const int i0 = ti * 32, j0 = tj * 32;
+    // this wave's edges [kb, ke)
+    const int per = ((K + KC - 1) / KC + 3) / 4 * KC, kb = min(K, w * per), ke = min(K, kb + per);
+    const double* x = wfc + (size_t)sim * nw * np + col0;
+    const double* src[4];
+    double mu[4], is[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {            // (rows past the last repeat it: their results are not kept)
+        const int row = min((q < 2 ? i0 + 16 * q : j0 + 16 * (q - 2)) + c, nw - 1);
+        src[q] = x + (size_t)row * np + V * g;
+        mu[q] = mean[(size_t)sim * nw + row];
+        is[q] = inv_ssd[(size_t)sim * nw + row];
+    }
+    V4 acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = V4{0, 0, 0, 0};
+    double ra[4][V], rb[4][V];
+    auto load = [&](double (&r)[4][V], int k) __attribute__((always_inline)) {
+        if (k + KC <= ke) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int s = 0; s < V; ++s) r[q][s] = src[q][k + s];
+        } else if (k < ke) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int s = 0; s < V; ++s) r[q][s] = k + V * g + s < ke ? src[q][k + s] : mu[q];   // z = 0
+        }
+    };
+    auto products = [&](const double (&r)[4][V]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < V; ++s) {
+            double z[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) z[q] = (r[q][s] - mu[q]) * is[q];
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) acc[a][b] = MF<double>::mma(z[a], z[2 + b], acc[a][b]);
+        }
+    };
+    load(ra, kb);
+    for (int k = kb; k < ke; k += 2 * KC) {
+        load(rb, k + KC);
+        __builtin_amdgcn_sched_barrier(0);
+        products(ra);
+        if (k + KC >= ke) break;
+        load(ra, k + 2 * KC);
+        __builtin_amdgcn_sched_barrier(0);
+        products(rb);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[(w * 16 + (2 * a + b) * 4 + r) * 64 + lane] = acc[a][b][r];
+    __syncthreads();
+    // wave w: 16 x 16 block (w / 2, w % 2)
+    double* out = fcd + (size_t)sim * ((long long)nw * (nw - 1) / 2);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        double v = 0;
+        for (int u = 0; u < 4; ++u) v += part[(u * 16 + w * 4 + r) * 64 + lane];
+        const int row = i0 + 16 * (w >> 1) + MF<double>::row(lane, r), col = j0 + 16 * (w & 1) + c;
+        if (row < nw && col < row) out[(long long)row * (row - 1) / 2 + col] = v;
+    }
+}
+
 template <class Tin, class Tc, class Tout>
 __global__ __launch_bounds__(256) void k_gram_fcd(const Tin* __restrict__ wfc, int nw, int np, int col0,
                                                   int K, const double* __restrict__ mean,
@@ -541,16 +653,47 @@ constexpr int ZLD32 = ZK32 + 4;   // floats per staged row (bank offset)
 constexpr int ZLDB = ZKB + 8;     // u16 per staged row
 }  // namespace
 
-template <int MODE>   // 0: FP32, 1: BF16, 2: BF16 hi + lo
-__global__ __launch_bounds__(256) void k_zscore_rows(const float* __restrict__ x, int np, int npp,
-                                                     const double* __restrict__ mean,
-                                                     const double* __restrict__ inv_ssd, void* __restrict__ zhi,
-                                                     unsigned short* __restrict__ zlo) {
+// A row of the window-FC matrix z-scored into Z, moments and all.  LDS: the row is
+// read once and kept there (each thread its own values); rows too long for that are
+// read three times.  Bound by memory: 18512 rows of 39800, 3.2 ms in two kernels (moments
+// read every row twice, then the z-scores once more) -> 2.1; a copy takes 1.25.
+template <int MODE, bool LDS>   // MODE 0: FP32, 1: BF16, 2: BF16 hi + lo
+__global__ __launch_bounds__(1024) void k_zrows(const float* __restrict__ x, int np, int npp, void* __restrict__ zhi,
+                                                unsigned short* __restrict__ zlo) {
+    extern __shared__ __align__(16) unsigned char zmem[];
+    __shared__ double red[16];
+    float* v = reinterpret_cast<float*>(zmem);
     const size_t row = blockIdx.x;
-    const double m = mean[row], is = inv_ssd[row];
     const float* r = x + row * np;
-    for (int i = threadIdx.x; i < npp; i += blockDim.x) {
-        const float z = i < np ? (float)(((double)r[i] - m) * is) : 0.0f;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    // f(i, value) for this thread's edges, four at a time
+    auto each = [&](const float* p, auto f) __attribute__((always_inline)) {
+        constexpr int U = 4;
+        int i = tid;
+        for (; i + (U - 1) * nt < np; i += U * nt) {
+            float a[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) a[u] = p[i + u * nt];
+#pragma unroll
+            for (int u = 0; u < U; ++u) f(i + u * nt, a[u]);
+        }
+        for (; i < np; i += nt) f(i, p[i]);
+    };
+    KSum s;
+    each(r, [&](int i, float a) __attribute__((always_inline)) {
+        if constexpr (LDS) v[i] = a;
+        s.add((double)a);
+    });
+    const float* own = LDS ? v : r;
+    const double tot = block_sum(s.s, red) + block_sum(s.c, red);
+    const double m = tot / np;
+    KSum q;
+    each(own, [&](int, float a) __attribute__((always_inline)) {
+        const double d = (double)a - m;
+        q.add(d * d);
+    });
+    const double is = 1.0 / sqrt(block_sum(q.s, red) + block_sum(q.c, red));
+    auto put = [&](int i, float z) __attribute__((always_inline)) {
         if constexpr (MODE == 0) {
             reinterpret_cast<float*>(zhi)[row * npp + i] = z;
         } else {
@@ -558,7 +701,9 @@ __global__ __launch_bounds__(256) void k_zscore_rows(const float* __restrict__ x
             reinterpret_cast<unsigned short*>(zhi)[row * npp + i] = h;
             if constexpr (MODE == 2) zlo[row * npp + i] = bf16_bits(z - __uint_as_float((unsigned)h << 16));
         }
-    }
+    };
+    each(own, [&](int i, float a) __attribute__((always_inline)) { put(i, (float)(((double)a - m) * is)); });
+    for (int i = np + tid; i < npp; i += nt) put(i, 0.0f);
 }
 
 // FP32 operands: tile rows ti*64.., tj*64.. of one simulation's Z
@@ -761,16 +906,26 @@ __global__ __launch_bounds__(256) void k_gram_z32_t128(const float* __restrict__
             }
 }
 
-hipError_t launch_fcd_z(const float* wfc, int B, int nw, int np, const double* mean, const double* inv_ssd,
-                        void* zhi, unsigned short* zlo, int mode, float* fcd, hipStream_t st, int tile) {
+namespace {
+template <int MODE>
+void launch_zrows(const float* wfc, unsigned rows, int np, int npp, void* zhi, unsigned short* zlo, hipStream_t st,
+                  size_t lds_max) {
+    const int threads = npp <= 4096 ? 256 : 1024;
+    const size_t lds = (size_t)np * sizeof(float);
+    if (lds + 256 <= lds_max)
+        hipLaunchKernelGGL((k_zrows<MODE, true>), dim3(rows), dim3(threads), lds, st, wfc, np, npp, zhi, zlo);
+    else
+        hipLaunchKernelGGL((k_zrows<MODE, false>), dim3(rows), dim3(threads), 0, st, wfc, np, npp, zhi, zlo);
+}
+}  // namespace
+
+hipError_t launch_fcd_z(const float* wfc, int B, int nw, int np, void* zhi, unsigned short* zlo, int mode, float* fcd,
+                        hipStream_t st, int tile, size_t lds_max) {
     const int npp = (np + 63) / 64 * 64;
     const unsigned rows = (unsigned)((long long)B * nw);
-    if (mode == 0)
-        hipLaunchKernelGGL(k_zscore_rows<0>, dim3(rows), dim3(256), 0, st, wfc, np, npp, mean, inv_ssd, zhi, zlo);
-    else if (mode == 1)
-        hipLaunchKernelGGL(k_zscore_rows<1>, dim3(rows), dim3(256), 0, st, wfc, np, npp, mean, inv_ssd, zhi, zlo);
-    else
-        hipLaunchKernelGGL(k_zscore_rows<2>, dim3(rows), dim3(256), 0, st, wfc, np, npp, mean, inv_ssd, zhi, zlo);
+    if (mode == 0) launch_zrows<0>(wfc, rows, np, npp, zhi, zlo, st, lds_max);
+    else if (mode == 1) launch_zrows<1>(wfc, rows, np, npp, zhi, zlo, st, lds_max);
+    else launch_zrows<2>(wfc, rows, np, npp, zhi, zlo, st, lds_max);
     const int nt = (nw + ZT - 1) / ZT;
     const dim3 grid(nt * (nt + 1) / 2, 1, B);
     const int nt2 = (nw + 127) / 128;
@@ -793,7 +948,7 @@ template <class T>
 hipError_t launch_seg_moments(const T* bold, int B, int N, int output_ts, int n_seg,
                               const int* seg_start, const int* seg_len, double* mean,
                               double* inv_ssd, hipStream_t st) {
-    hipLaunchKernelGGL(k_seg_moments<T>, dim3((unsigned)(((long long)n_seg * N + 255) / 256), B), dim3(256), 0, st, bold, N, output_ts,
+    hipLaunchKernelGGL(k_seg_moments<T>, dim3((unsigned)(((long long)n_seg * N + 63) / 64), B), dim3(256), 0, st, bold, N, output_ts,
                        n_seg, seg_start, seg_len, mean, inv_ssd);
     return hipGetLastError();
 }
@@ -835,9 +990,15 @@ template <class Tin, class Tc, class Tout>
 hipError_t launch_gram_fcd(const Tin* wfc, int B, int nw, int np, const double* mean,
                            const double* inv_ssd, Tout* fcd, hipStream_t st, int col0, int K) {
     if (K < 0) K = np;
-    const int nt = (nw + TM - 1) / TM;
-    hipLaunchKernelGGL((k_gram_fcd<Tin, Tc, Tout>), dim3(nt * (nt + 1) / 2, 1, B), dim3(256), 0, st,
-                       wfc, nw, np, col0, K, mean, inv_ssd, fcd);
+    if constexpr (sizeof(Tc) == 8) {
+        const int n = (nw + 31) / 32, tiles = n * (n + 1) / 2, total = tiles * B;
+        hipLaunchKernelGGL(k_gram_fcd64, dim3(xcd_grid(total)), dim3(256), 0, st, wfc, nw, np, col0, K, mean, inv_ssd,
+                           tiles, total, fcd);
+    } else {
+        const int nt = (nw + TM - 1) / TM;
+        hipLaunchKernelGGL((k_gram_fcd<Tin, Tc, Tout>), dim3(nt * (nt + 1) / 2, 1, B), dim3(256), 0, st,
+                           wfc, nw, np, col0, K, mean, inv_ssd, fcd);
+    }
     return hipGetLastError();
 }
 
