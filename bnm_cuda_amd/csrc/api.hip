@@ -1228,8 +1228,8 @@ static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only
     if (!c.sim_only && !c.no_fcd) {
         HIPCHK(launch_fill_i32(x->bins, (long long)x->B * (2 * x->m + 1), 0, st));
         HIPCHK(launch_fill_i32(x->nanf, x->B, 0, st));
-        if (x->fc64) HIPCHK(launch_ks_bin<double>((const double*)x->fcd, g, st));
-        else HIPCHK(launch_ks_bin<float>((const float*)x->fcd, g, st));
+        if (x->fc64) HIPCHK(launch_ks_bin<double>((const double*)x->fcd, g, st, x->lds_max));
+        else HIPCHK(launch_ks_bin<float>((const float*)x->fcd, g, st, x->lds_max));
     }
     if (x->fc64) HIPCHK(launch_gof<double>((const double*)x->fc, g, st));
     else HIPCHK(launch_gof<float>((const float*)x->fc, g, st));

@@ -197,7 +197,7 @@ struct GofArgs {
     double* fic_pen;             // [B]
 };
 template <class T>
-hipError_t launch_ks_bin(const T* fcd, const GofArgs& g, hipStream_t st);
+hipError_t launch_ks_bin(const T* fcd, const GofArgs& g, hipStream_t st, size_t lds_max);
 template <class T>
 hipError_t launch_gof(const T* fc, const GofArgs& g, hipStream_t st);
 hipError_t launch_fill_i32(int* p, long long n, int v, hipStream_t st);
