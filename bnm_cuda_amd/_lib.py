@@ -30,7 +30,7 @@ EXPORTS = (
     "bnm_default_config", "bnm_finalize_config", "bnm_output_ts", "bnm_n_pairs", "bnm_n_windows",
     "bnm_window_bounds", "bnm_regional_params", "bnm_analytical_fic", "bnm_make_noise", "bnm_make_noise_chunked", "bnm_sparse_layout", "bnm_run_simulations", "bnm_run_simulations_noalloc", "bnm_ctx_create",
     "bnm_ctx_destroy", "bnm_ctx_set_sc", "bnm_ctx_set_noise", "bnm_ctx_set_empirical",
-    "bnm_ctx_set_params", "bnm_ctx_run", "bnm_ctx_set_bold", "bnm_ctx_analyze", "bnm_ctx_get_hemi_fcd", "bnm_ctx_get_outputs", "bnm_ctx_timings",
+    "bnm_ctx_set_params", "bnm_ctx_run", "bnm_ctx_set_bold", "bnm_ctx_analyze", "bnm_ctx_get_hemi_fcd", "bnm_ctx_get_outputs", "bnm_ctx_get_ext", "bnm_ctx_timings",
     "bnm_ctx_kernel_name", "bnm_ctx_tune_log", "bnm_multi_create", "bnm_multi_run",
     "bnm_multi_last_ms", "bnm_multi_plan", "bnm_multi_destroy", "bnm_cmaes_create", "bnm_cmaes_destroy",
     "bnm_cmaes_ask", "bnm_cmaes_tell", "bnm_cmaes_best", "bnm_cmaes_sigma", "bnm_cmaes_strategy", "bnm_cmaes_iteration", "bnm_cmaes_ask_pool", "bnm_cmaes_select",
@@ -104,6 +104,7 @@ def lib():
     L.bnm_ctx_set_bold.argtypes = [vp, pd]
     L.bnm_ctx_analyze.argtypes = [vp]
     L.bnm_ctx_get_hemi_fcd.argtypes = [vp, pd, pd]
+    L.bnm_ctx_get_ext.argtypes = [vp, pd]
     L.bnm_ctx_get_outputs.argtypes = [vp, pd, pd, pd] + [pd] * 7 + [pi, pi, pd, pd]
     L.bnm_ctx_timings.argtypes = [vp, pd, C.c_int]
     L.bnm_ctx_kernel_name.argtypes = [vp]
@@ -347,19 +348,18 @@ class Context:
     def outputs(self, bold=True, fc=True, fcd=True):
         B, N = self.B, self.N
         o = dict(corr=np.zeros(B), fic_penalty=np.zeros(B), wIE_fic=np.zeros((B, N)),
-                 ext=np.zeros((6, B, N)), fic_failed=np.zeros(B, np.int32),
+                 ext=np.zeros((B, 6, N)), fic_failed=np.zeros(B, np.int32),
                  fic_trials=np.zeros(B, np.int32))
         o["bold"] = np.zeros((B, self.ots, N)) if bold else None
         o["fc"] = np.zeros((B, self.np)) if (fc and self.np) else None
         o["fcd"] = np.zeros((B, self.nwp)) if (fcd and self.nwp) else None
-        e = o["ext"]
         _chk(lib().bnm_ctx_get_outputs(
             self.h, _p(o["corr"], C.c_double), _p(o["fic_penalty"], C.c_double),
             _p(o["wIE_fic"], C.c_double), _p(o["bold"], C.c_double),
-            *[_p(e[i], C.c_double) for i in range(6)],
+            *[None] * 6,
             _p(o["fic_failed"], C.c_int), _p(o["fic_trials"], C.c_int),
             _p(o["fc"], C.c_double), _p(o["fcd"], C.c_double)))
-        o["ext"] = np.ascontiguousarray(np.transpose(e, (1, 0, 2)))  # [B][6][N]
+        _chk(lib().bnm_ctx_get_ext(self.h, _p(o["ext"], C.c_double)))
         o["fic_failed"] = o["fic_failed"].astype(bool)
         return o
 

@@ -242,6 +242,9 @@ int bnm_ctx_get_outputs(bnm_ctx* ctx, double* corr, double* fic_penalties, doubl
                         double* BOLD, double* S_E, double* I_E, double* r_E, double* S_I,
                         double* I_I, double* r_I, int* FIC_failed, int* fic_n_trials,
                         double* fc_trils, double* fcd_trils);
+/* The six averages as they lie on the device, [B][S_E I_E r_E S_I I_I r_I][N]:
+ * one copy instead of six arrays. */
+int bnm_ctx_get_ext(bnm_ctx* ctx, double* ext);
 /* Left and right FCD [B*n_window_pairs] of the last run (save_hemis): the
  * reference's save_hemis outputs L_fcd_trils / R_fcd_trils (bnm.cu:498-550),
  * with n_pairs_hemi = (N/2)(N/2-1)/2.  With exc_interhemispheric on, the
