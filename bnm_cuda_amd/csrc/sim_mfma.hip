@@ -3,15 +3,24 @@
 //   C[N x 16] = SC[N x N] . S_E[N x 16]
 // (bnm.cu:186-189 computes the same dot per node and simulation).
 //
-// Workgroup = 16 simulations; wave w owns the 16-node row tile w (N <= 128,
-// so at most 8 waves).  Lane l of wave w holds the MFMA output rows
-// 4*(l/16)..+3 of column l%16, i.e. four (node, simulation) pairs, and keeps
-// their state in registers for the whole run.  SC row tiles are loaded once
-// into VGPRs as A fragments; S_E of the 16 simulations is double-buffered in
-// LDS as [sim][k] rows (padded so a 16-lane group's 16-byte reads hit distinct
-// banks) and read as B fragments.  The K axis is permuted so that lane group
-// g = l/16 supplies the contiguous k-range [g*KQ, (g+1)*KQ), which lets every
-// B fragment come from one vector load.
+// Workgroup = 16 simulations, one wave a SIMD (N <= 64) or two (N <= 128).  The
+// nodes are dealt to the waves in quads, q = 1..4 a wave: lane l of a wave holds q
+// (node, simulation) pairs, the first q of its four MFMA output rows 4*(l/16)..+3
+// of column l%16 (the other rows of the tile are zero), and keeps their state in
+// registers for the whole run.  SC row tiles are loaded once into VGPRs as A
+// fragments; S_E of the 16 simulations is double-buffered in LDS as [sim][k] rows
+// (padded so a 16-lane group's 16-byte reads hit distinct banks) and read as B
+// fragments.  Lane group g = l/16 supplies k = 4 step + g (FP32; a row holds each
+// group's values together) or the contiguous k-range [g*KQ, (g+1)*KQ) (BF16), so
+// that every B fragment comes from vector loads.
+//
+// Bound (N = 100, 4096 simulations, FP32; one workgroup a CU): 3660 cycles a substep,
+// of which the products of a SIMD's two waves 2 x 25 x 32 in its matrix pipe, two
+// waves' updates of four and three sets of ~40 instructions, and LDS and the barrier;
+// the phases hardly overlap (wave priorities and a second chain of products change
+// nothing).  It was 5000: seven tiles of 16 rows put eight sets on three SIMDs and
+// four on the last, K was padded to 128, and each substep's noise was waited for in
+// that substep.  62.3 -> 45.3 ms for 3 s.
 //
 // MODE 0  FP32 operands, v_mfma_f32_16x16x4_f32
 // MODE 1  BF16 operands, v_mfma_f32_16x16x32_bf16, FP32 accumulate
@@ -22,6 +31,7 @@
 // per-simulation durations are independent; finished simulations idle.
 #include "kernels.hpp"
 #include "model.hpp"
+#include "pool.hpp"
 
 namespace bnm {
 
@@ -46,15 +56,18 @@ constexpr int kSims = 16;
 template <int MODE, int KQ>
 __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, SimArgs a,
                                                   int n_sims_total, int LDSS) {
-    static_assert(KQ % 8 == 0, "KQ must be a multiple of 8");
+    static_assert(KQ % (MODE == 0 ? 4 : 8) == 0, "KQ must be a multiple of the vector of a B fragment");
     constexpr int NSTEP = MODE == 0 ? KQ : KQ / 8;  // MFMA steps per row tile
     const int N = a.N;
-    const int lane = threadIdx.x & 63, rt = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, rt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int sim = blockIdx.x * kSims + n;
     const bool sim_ok = sim < n_sims_total;
-    const int row_a = rt * 16 + n;            // A-fragment row of this lane
-    const int j0 = rt * 16 + 4 * g;           // first of this lane's 4 output nodes
+    // this wave's nodes: q a lane, 4 q from j_w on
+    const int quads = (N + 3) / 4, W = blockDim.x >> 6;
+    const int q = quads / W + (rt < quads % W ? 1 : 0), j_w = 4 * (rt * (quads / W) + min(rt, quads % W));
+    const int row_a = (n & 3) < q ? j_w + (n >> 2) * q + (n & 3) : N;   // A-fragment row of this lane (N: none)
+    const int j0 = j_w + g * q;               // first of this lane's q output nodes
 
     extern __shared__ unsigned char smem_raw[];
     // FP32 mode: float S[2][16][LDSS]; BF16 modes: u16 hi[2][16][LDSS], lo[2][16][LDSS]
@@ -70,7 +83,7 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
     if constexpr (MODE == 0) {
 #pragma unroll
         for (int kk = 0; kk < KQ; ++kk) {
-            const int k = g * KQ + kk;
+            const int k = 4 * kk + g;
             a32[kk] = (row_a < N && k < N) ? SC[(size_t)row_a * N + k] : 0.0f;
         }
     } else {
@@ -88,7 +101,8 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
     // ---- LDS init: S_E = 0.001 on real nodes, 0 on padding ----------------
     const int nbuf = 2 * kSims * LDSS;
     for (int i = threadIdx.x; i < nbuf; i += blockDim.x) {
-        const int k = i % LDSS;
+        int k = i % LDSS;
+        if (MODE == 0) k = k < 4 * KQ ? 4 * (k % KQ) + k / KQ : N;   // (see at())
         const float v = k < N ? 0.001f : 0.0f;
         if constexpr (MODE == 0) {
             S32[i] = v;
@@ -100,6 +114,9 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
     }
     if (threadIdx.x < kSims) flags[threadIdx.x] = 0;
 
+    // where S_E of node j lies in its simulation's row: FP32, what lane group g takes
+    // in consecutive steps (nodes 4 step + g) together; BF16, in order
+    auto at = [](int j) { return MODE == 0 ? (j & 3) * KQ + (j >> 2) : j; };
     // ---- per-pair state ---------------------------------------------------
     bool node_ok[4];
     float SE[4], SI[4], IE[4], II[4], rE[4], rI[4], wEE[4], wEI[4], wIE[4], delta[4];
@@ -110,7 +127,7 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int j = j0 + r;
-        node_ok[r] = sim_ok && j < N;
+        node_ok[r] = sim_ok && r < q && j < N;
         const size_t o = (size_t)sim * N + j;
         SE[r] = 0.001f; SI[r] = 0.001f;
         IE[r] = II[r] = rE[r] = rI[r] = 0.0f;
@@ -127,26 +144,38 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
     const unsigned dur = (unsigned)(a.i_end - a.i_start + 1);
     const int P = (int)a.noise_period;
     const float2* noise2 = reinterpret_cast<const float2*>(a.noise);
-    int buf = 0;
+    constexpr int buf0 = 0;   // (ten substeps a ms: each starts with the same S_E buffer)
+    // Noise of the lane's nodes, two substeps ahead (memory's latency is about half a
+    // substep's time, and loads return in order), without conditions, so that the
+    // waits can be counted: nodes past the last take the last one's.
+    constexpr int kAhead = 5;
+    float2 nzb[kAhead][4];
+    int jn[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) jn[r] = min(j0 + r, N - 1);
+    auto noise_of = [&](float2 (&to)[4], const float2* p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) to[r] = p[jn[r]];
+    };
+    auto noise_first = [&]() __attribute__((always_inline)) {
+        const float2* p = noise2 + (size_t)(ts % P) * 10 * N;
+        noise_of(nzb[0], p);
+        noise_of(nzb[1], p + N);
+    };
+    noise_first();
     __syncthreads();
 
     while (__syncthreads_or(sim_ok && ts <= T)) {
         const bool active = sim_ok && ts <= T;
-        const int ms = ts % P;
-        const float2* nzp = noise2 + (size_t)ms * 10 * N + j0;
-        // noise of the lane's four nodes, one substep ahead: the loads for
-        // substep s + 1 are in flight behind substep s
-        float2 nz[4], nzn[4];
+        const float2* nz_now = noise2 + (size_t)(ts % P) * 10 * N;
+        const float2* nz_next = noise2 + (size_t)((ts + 1) % P) * 10 * N;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) nzn[r] = node_ok[r] && active ? nzp[r] : float2{0, 0};
         for (int s = 0; s < 10; ++s) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) nz[r] = nzn[r];
-            if (s < 9) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    nzn[r] = node_ok[r] && active ? nzp[(size_t)(s + 1) * N + r] : float2{0, 0};
-            }
+            const int buf = buf0 ^ (s & 1);
+            float2 (&nz)[4] = nzb[s % kAhead];
+            __builtin_amdgcn_sched_barrier(0);
+            noise_of(nzb[(s + 2) % kAhead], s + 2 < 10 ? nz_now + (s + 2) * N : nz_next + (s + 2 - 10) * N);
+            __builtin_amdgcn_sched_barrier(0);
             // ---- coupling on MFMA ------------------------------------------
             f32x4 acc = {0, 0, 0, 0};
             if constexpr (MODE == 0) {
@@ -157,8 +186,10 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
 #pragma unroll
                 for (int q = 0; q < KQ / 4; ++q)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
+                    for (int e = 0; e < 4; ++e) {
+                        if (q == KQ / 4 - 1 && e > 0 && 4 * q + e >= quads) continue;   // (the last vector's padding)
                         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a32[4 * q + e], bv[q][e], acc, 0, 0, 0);
+                    }
             } else {
                 const u16x8* Bh = reinterpret_cast<const u16x8*>(Shi + (buf * kSims + n) * LDSS + g * KQ);
                 const u16x8* Bl = reinterpret_cast<const u16x8*>(Slo + (buf * kSims + n) * LDSS + g * KQ);
@@ -181,30 +212,21 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
             if (active) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (node_ok[r])
+                    if (node_ok[r]) {
                         Node<float>::step(acc[r], gj, wEE[r], wEI[r], wIE[r], nz[r].x, nz[r].y, SE[r],
                                           SI[r], IE[r], II[r], rE[r], rI[r]);
-                const int base = ((buf ^ 1) * kSims + n) * LDSS + j0;
-                if (j0 < N) {
-                    if constexpr (MODE == 0) {
-                        f32x4 v;
-                        for (int r = 0; r < 4; ++r) v[r] = node_ok[r] ? SE[r] : 0.0f;
-                        *reinterpret_cast<f32x4*>(S32 + base) = v;
-                    } else {
-                        u16x4 h, l;
-                        for (int r = 0; r < 4; ++r) {
-                            const float v = node_ok[r] ? SE[r] : 0.0f;
-                            h[r] = f2bf(v);
-                            l[r] = f2bf(v - bf2f(h[r]));
+                        const int o = ((buf ^ 1) * kSims + n) * LDSS + at(j0 + r);
+                        if constexpr (MODE == 0) {
+                            S32[o] = SE[r];
+                        } else {
+                            const unsigned short h = f2bf(SE[r]);
+                            Shi[o] = h;
+                            if constexpr (MODE == 2) Slo[o] = f2bf(SE[r] - bf2f(h));
                         }
-                        *reinterpret_cast<u16x4*>(Shi + base) = h;
-                        if constexpr (MODE == 2) *reinterpret_cast<u16x4*>(Slo + base) = l;
                     }
-                }
             }
             // (a finished simulation's column is independent of the others)
-            __syncthreads();
-            buf ^= 1;
+            lds_barrier();
         }
         if (active) {
 #pragma unroll
@@ -251,19 +273,17 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
                             bw[r].reset();
                             for (int e = 0; e < 6; ++e) ext[r][e] = 0.0f;
                         }
-                        if (j0 < N) {
-                            const int base = (buf * kSims + n) * LDSS + j0;
-                            for (int r = 0; r < 4; ++r) {
-                                const float v = node_ok[r] ? 0.001f : 0.0f;
+                        const int base = (buf0 * kSims + n) * LDSS;
+                        for (int r = 0; r < 4; ++r)
+                            if (node_ok[r]) {
                                 if constexpr (MODE == 0) {
-                                    S32[base + r] = v;
+                                    S32[base + at(j0 + r)] = 0.001f;
                                 } else {
-                                    const unsigned short h = f2bf(v);
-                                    Shi[base + r] = h;
-                                    if constexpr (MODE == 2) Slo[base + r] = f2bf(v - bf2f(h));
+                                    const unsigned short h = f2bf(0.001f);
+                                    Shi[base + at(j0 + r)] = h;
+                                    if constexpr (MODE == 2) Slo[base + at(j0 + r)] = f2bf(0.001f - bf2f(h));
                                 }
                             }
-                        }
                         ts = 0; vol = 0; ++trial;
                     } else {
                         failed = true; adjusting = false;
@@ -272,6 +292,7 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
                     adjusting = false;
                 }
             }
+            noise_first();
             __syncthreads();
         }
     }
@@ -294,9 +315,10 @@ __global__ __launch_bounds__(512) void k_sim_mfma(const float* __restrict__ SC, 
 MfmaShape mfma_shape(int N, int mode) {
     MfmaShape s{};
     s.mode = mode;
-    const int KP = ((N + 31) / 32) * 32;
+    const int kp = mode == 0 ? 16 : 32, KP = (N + kp - 1) / kp * kp;
     s.KQ = KP / 4;
-    s.waves = (N + 15) / 16;
+    // One wave a SIMD, or two: the nodes in quads over all of them
+    s.waves = N <= 64 ? 4 : 8;
     s.threads = s.waves * 64;
     // row stride of the LDS S_E rows: KP + pad, chosen so that (stride in
     // dwords) mod 32 == 4 and a 16-lane group's 16-byte reads are conflict-free
@@ -305,18 +327,27 @@ MfmaShape mfma_shape(int N, int mode) {
     while (((ld * el / 4) % 32) != 4) ld += 16 / el;
     s.LDSS = ld;
     s.smem = (size_t)(mode == 0 ? 2 : 4) * kSims * ld * el + kSims * sizeof(int);
-    s.ok = N <= 128 && (mode >= 0 && mode <= 2) && (s.KQ == 8 || s.KQ == 16 || s.KQ == 24 || s.KQ == 32);
+    s.ok = N <= 128 && mode >= 0 && mode <= 2;
     return s;
 }
 
 template <int MODE>
 static void launch_mode(const float* SC, const SimArgs& a, const MfmaShape& s, hipStream_t st) {
     const dim3 grid((a.B + kSims - 1) / kSims);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(s.threads), s.smem, st, SC, a, a.B, s.LDSS);
+    };
     switch (s.KQ) {
-        case 8: hipLaunchKernelGGL((k_sim_mfma<MODE, 8>), grid, dim3(s.threads), s.smem, st, SC, a, a.B, s.LDSS); break;
-        case 16: hipLaunchKernelGGL((k_sim_mfma<MODE, 16>), grid, dim3(s.threads), s.smem, st, SC, a, a.B, s.LDSS); break;
-        case 24: hipLaunchKernelGGL((k_sim_mfma<MODE, 24>), grid, dim3(s.threads), s.smem, st, SC, a, a.B, s.LDSS); break;
-        default: hipLaunchKernelGGL((k_sim_mfma<MODE, 32>), grid, dim3(s.threads), s.smem, st, SC, a, a.B, s.LDSS); break;
+        case 8: return go(k_sim_mfma<MODE, 8>);
+        case 16: return go(k_sim_mfma<MODE, 16>);
+        case 24: return go(k_sim_mfma<MODE, 24>);
+        case 32: return go(k_sim_mfma<MODE, 32>);
+    }
+    if constexpr (MODE == 0) switch (s.KQ) {
+        case 4: return go(k_sim_mfma<0, 4>);
+        case 12: return go(k_sim_mfma<0, 12>);
+        case 20: return go(k_sim_mfma<0, 20>);
+        case 28: return go(k_sim_mfma<0, 28>);
     }
 }
 
