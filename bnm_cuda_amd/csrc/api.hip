@@ -1029,7 +1029,18 @@ static std::vector<Variant> candidates(const bnm_ctx* x) {
         for (const Variant& v : out) hyb = hyb || v.kind == 5 || v.kind == 7;
         if (hyb) out.erase(std::remove_if(out.begin(), out.end(), [](const Variant& v) { return v.kind == 1; }), out.end());
         std::stable_partition(out.begin(), out.end(), [](const Variant& v) { return v.kind == 8; });
-        if (x->gang_mode != 0) add({10, 1, 1, 0});
+        // ...as long as all members are resident at once (a workgroup a CU, each
+        // simulation on one XCD): members of a second round start one by one, as
+        // simulations of the first end, and wait for each other in vain when those
+        // end at different times (FP64, 128 simulations of N = 400, 2.7 s with FIC:
+        // 0.64 s with the launch that takes over, 0.48 on one workgroup each, though
+        // the tuner's window of equal lengths says 24 against 53 ms)
+        int cus = 256, dev = 0, v = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+            cus = v;
+        const bool resident = (x->B + 7) / 8 * gang_shape(x->N, x->f64 ? 8 : 4).C <= cus / 8;
+        if (x->gang_mode > 0 || (x->gang_mode != 0 && resident)) add({10, 1, 1, 0});
     }
     // the MFMA kernel implements FP32 too; the tuner may pick it for large populations
     if (c.kernel == BNM_KERNEL_AUTO && !x->f64 && !pinned && !x->force_stream) add({2, 0, 0, 0});

@@ -11,8 +11,9 @@
 //
 // Exchange: one 64-bit word per node (FP32; two for FP64, 32 bits each) holds
 // the new S_E and the number of its substep: a word is its own flag, so no
-// fence is needed.  A poll reads two words (16 bytes), each checked by itself.  The members of a simulation get block indices 8 apart, i.e.
-// one XCD, and meet in its L2: a plain store (the L1 writes through) is seen by a
+// fence is needed.  A poll reads two words (16 bytes), each checked by itself.
+// The members of a simulation get block indices 8 apart, i.e. one XCD, and meet in
+// its L2: a plain store (the L1 writes through) is seen by a
 // poll that passes the L1 by (agent scope) 0.27 us later; a store of agent scope
 // goes on to memory and takes 0.39 us.  That the members do share an XCD is
 // checked when they start.  Words are double-buffered by substep parity; a
