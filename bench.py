@@ -11,8 +11,8 @@ N(0,1) float draws covering the whole run (seed 1); empirical target = FC/FCD
 of the single-simulation config (G 0.5, wEE 0.21, wEI 0.15) on a second SC
 (seed 2), simulated once by the FP64 path before timing.
 
-A step is one bnm_ctx_run: analytical FIC, integration (FP32 register-resident
-split kernel), FC, windowed FC, FCD and the KS fit for all 128 simulations, on
+A step is one bnm_ctx_run: analytical FIC, integration (FP32 row-blocked
+kernel), FC, windowed FC, FCD and the KS fit for all 128 simulations, on
 inputs already resident in HBM.  `value` counts nominal simulated seconds
 (128 x 450 s per step); FIC restarts re-simulate 10 s each and are reported
 separately.
@@ -42,11 +42,11 @@ PEAK_HBM_GBS = 8000.0
 # from two rocprofv3 --pmc passes over `bench.py --steps 1 --warmup 0
 # --no-fp64 --no-cpu --no-extras` (FETCH_SIZE, then WRITE_SIZE, KiB per
 # dispatch), each scaled by what the counter reads for a 1 GiB device copy
-# (FETCH_SIZE reads 0.5x, WRITE_SIZE 1.0x): 79,399,407.5 KiB x 2 fetched +
-# 26,524.4 KiB written by the strict E/I kernel.  Valid for the split_ei
-# kernel family at 128 x 450 s; other shapes report null.
-MEASURED_TRAFFIC = {"kernel_prefix": "split_ei_f32", "n_sims": 128, "duration_ms": 450_000,
-                    "bytes": int(79_399_407.5 * 1024 * 2 + 26_524.4 * 1024)}
+# (FETCH_SIZE reads 0.5x, WRITE_SIZE 1.0x): 79,053,875.9 KiB x 2 fetched +
+# 26,524.4 KiB written by the row-blocked kernel.  Valid for that kernel
+# at 128 x 450 s; other shapes report null.
+MEASURED_TRAFFIC = {"kernel_prefix": "block_f32", "n_sims": 128, "duration_ms": 450_000,
+                    "bytes": int(79_053_875.9 * 1024 * 2 + 26_524.4 * 1024)}
 
 
 def log(*a):
