@@ -158,6 +158,7 @@ struct bnm_ctx {
     double solo_ms_per_sim_ms = -1;
     unsigned long long* gang = nullptr;   // exchange words of kind 10
     int gang_mode = -1, gang_polls = kGangStartPolls;
+    int cus = 256;
     hipGraphExec_t graph_exec = nullptr;
     bool have_sc = false, have_noise = false, have_emp = false, have_params = false;
     int fast_ls = 0, fast_ks = 0, stream_ks = 0, force_stream = 0, no_ei = 0, ei_ls = 0, ei_bc = 0, ei_form = -1, no_hyb = 0, hyb_ks = 0, hyb_bc = -1, hyb_rr = -1;
@@ -629,6 +630,7 @@ static bnm_ctx* ctx_create(const bnm_config* cfg, int* status, unsigned char* ar
         if (hipGetDevice(&dev) == hipSuccess &&
             hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 0)
             x->lds_max = (size_t)v;
+        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) x->cus = v;
     }
     x->autotune = c.autotune;
     x->tune_ms = env_int("BNM_TUNE_MS", 300);
@@ -898,8 +900,8 @@ static hipError_t launch_variant(bnm_ctx* x, const Variant& v, const SimArgs& a,
                                      x->lds_max, st);
         case 9: return x->f64 ? launch_sim_block<double>(x->SC64, a, st) : launch_sim_block<float>(x->SC32, a, st);
         case 10: {
-            const hipError_t e = x->f64 ? launch_sim_gang<double>(x->SC64, a, x->gang, x->gang_polls, st)
-                                        : launch_sim_gang<float>(x->SC32, a, x->gang, x->gang_polls, st);
+            const hipError_t e = x->f64 ? launch_sim_gang<double>(x->SC64, a, x->gang, x->gang_polls, x->cus, st)
+                                        : launch_sim_gang<float>(x->SC32, a, x->gang, x->gang_polls, x->cus, st);
             if (e != hipSuccess) return e;
             SimArgs b = a;
             b.only = gang_state(x->gang, x->N, x->B, x->f64 ? 8 : 4);
@@ -1029,18 +1031,7 @@ static std::vector<Variant> candidates(const bnm_ctx* x) {
         for (const Variant& v : out) hyb = hyb || v.kind == 5 || v.kind == 7;
         if (hyb) out.erase(std::remove_if(out.begin(), out.end(), [](const Variant& v) { return v.kind == 1; }), out.end());
         std::stable_partition(out.begin(), out.end(), [](const Variant& v) { return v.kind == 8; });
-        // ...as long as all members are resident at once (a workgroup a CU, each
-        // simulation on one XCD): members of a second round start one by one, as
-        // simulations of the first end, and wait for each other in vain when those
-        // end at different times (FP64, 128 simulations of N = 400, 2.7 s with FIC:
-        // 0.64 s with the launch that takes over, 0.48 on one workgroup each, though
-        // the tuner's window of equal lengths says 24 against 53 ms)
-        int cus = 256, dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-            cus = v;
-        const bool resident = (x->B + 7) / 8 * gang_shape(x->N, x->f64 ? 8 : 4).C <= cus / 8;
-        if (x->gang_mode > 0 || (x->gang_mode != 0 && resident)) add({10, 1, 1, 0});
+        if (x->gang_mode != 0) add({10, 1, 1, 0});
     }
     // the MFMA kernel implements FP32 too; the tuner may pick it for large populations
     if (c.kernel == BNM_KERNEL_AUTO && !x->f64 && !pinned && !x->force_stream) add({2, 0, 0, 0});

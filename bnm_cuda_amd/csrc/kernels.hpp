@@ -100,6 +100,7 @@ hipError_t launch_sim_block(const T* SC, const SimArgs& a, hipStream_t st);
 constexpr int kGangMembers = 16, kGangThreads = 512, kGangStartPolls = 1 << 16;
 struct GangArgs {
     int C;                         // workgroups per simulation
+    int groups;                    // of C workgroups on each XCD
     int start_polls;               // polls of ~0.5 us that a workgroup waits for the others
     unsigned long long* xch;       // [B][2][words of a row]
     unsigned long long* flag;      // [B][kGangMembers]
@@ -114,7 +115,8 @@ GangShape gang_shape(int N, size_t elem);
 size_t gang_words(int N, int B, size_t elem);
 const unsigned long long* gang_state(const unsigned long long* words, int N, int B, size_t elem);
 template <class T>
-hipError_t launch_sim_gang(const T* SC, const SimArgs& a, unsigned long long* words, int start_polls, hipStream_t st);
+hipError_t launch_sim_gang(const T* SC, const SimArgs& a, unsigned long long* words, int start_polls, int cus,
+                           hipStream_t st);
 template <class R>
 hipError_t launch_sim_stream(const R* SCt, const SimArgs& a, int KS, hipStream_t st);
 

@@ -28,7 +28,11 @@
 // follows in the stream (SimArgs::only) runs the marked simulations on one
 // workgroup each.  From then on all members are resident, and the polls in the
 // time loop end when the others get there; they have a bound too (kLoopPolls),
-// with the same consequence.
+// with the same consequence.  A group of members runs one simulation after the other,
+// as many groups as have a CU for each member: members of a second round of
+// workgroups would start one by one, as simulations of the first end, and wait in
+// vain for each other (FP64, 128 simulations of N = 400 with FIC, 2.7 s: 0.64 s with
+// the launch that takes over, 0.48 on one workgroup each, 0.22 with groups).
 //
 // What bounds it: the exchange.  At N = 400 (FP32, 16 simulations on 112 CUs) one
 // substep is 1810 cycles: 850 from store to the value in the others' LDS, 450 of
@@ -95,8 +99,11 @@ __device__ __forceinline__ T gang_sum(T (&acc)[2]) {
 
 }  // namespace
 
+// one simulation on the C workgroups of a group; every thread of a member returns
+// after the same number of barriers
 template <class T, int R, int KC>
-__global__ __launch_bounds__(kGangThreads) void k_sim_gang(const T* __restrict__ SC, SimArgs a, GangArgs ga, int SS) {
+__device__ __forceinline__ void gang_run(const T* __restrict__ SC, const SimArgs& a, const GangArgs& ga, int SS,
+                                         int member, int sim) {
     constexpr bool F64 = sizeof(T) == 8;
     constexpr int WPV = sizeof(T) / 4;             // exchange words per node
     constexpr int NPU = 2 / WPV;                    // nodes in the 16 bytes of a poll
@@ -106,8 +113,6 @@ __global__ __launch_bounds__(kGangThreads) void k_sim_gang(const T* __restrict__
     constexpr int VW = 16 / sizeof(T);
     typedef T vec __attribute__((ext_vector_type(VW)));
     const int C = ga.C;
-    const int member = (blockIdx.x >> 3) % C, sim = (blockIdx.x >> 3) / C * 8 + (blockIdx.x & 7);
-    if (sim >= a.B) return;
     const int N = a.N, tid = threadIdx.x & 255, threads = kGangThreads;
     const bool poller = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) != 0;
     const int lane = tid & 63, q = lane & 15, pop = lane & 1;
@@ -423,6 +428,17 @@ __global__ __launch_bounds__(kGangThreads) void k_sim_gang(const T* __restrict__
     }
 }
 
+// A group of members takes one simulation after the other, so that all members are
+// resident from the start, whatever the population: a workgroup a CU.
+template <class T, int R, int KC>
+__global__ __launch_bounds__(kGangThreads) void k_sim_gang(const T* __restrict__ SC, SimArgs a, GangArgs ga, int SS) {
+    const int member = (blockIdx.x >> 3) % ga.C;
+    for (int sim = (blockIdx.x >> 3) / ga.C * 8 + (blockIdx.x & 7); sim < a.B; sim += 8 * ga.groups) {
+        gang_run<T, R, KC>(SC, a, ga, SS, member, sim);
+        __syncthreads();
+    }
+}
+
 // FP32: N of 257 to 512, R = 4 (64 nodes a member).  FP64: 129 to 256 with R = 4,
 // to 512 with R = 2 (32 nodes a member: R x KC doubles are the same VGPRs).
 static const int kGangKC[] = {10, 13, 16, 20, 25, 28, 32};
@@ -451,18 +467,20 @@ size_t gang_words(int N, int B, size_t elem) {
 
 template <class T, int R, int KC>
 static void launch_gang(const T* SC, const SimArgs& a, const GangArgs& g, const GangShape& s, hipStream_t st) {
-    hipLaunchKernelGGL((k_sim_gang<T, R, KC>), dim3(8 * s.C * ((a.B + 7) / 8)), dim3(kGangThreads), s.smem, st, SC, a,
+    hipLaunchKernelGGL((k_sim_gang<T, R, KC>), dim3(8 * s.C * g.groups), dim3(kGangThreads), s.smem, st, SC, a,
                        g, s.SS);
 }
 
 template <class T>
-hipError_t launch_sim_gang(const T* SC, const SimArgs& a, unsigned long long* words, int start_polls, hipStream_t st) {
+hipError_t launch_sim_gang(const T* SC, const SimArgs& a, unsigned long long* words, int start_polls, int cus,
+                           hipStream_t st) {
     const GangShape s = gang_shape(a.N, sizeof(T));
     if (!s.ok) return hipErrorInvalidValue;
     GangArgs g{};
     g.C = s.C;
     g.start_polls = start_polls;
     g.xch = words;
+    g.groups = std::max(1, std::min((a.B + 7) / 8, cus / 8 / s.C));   // per XCD
     g.flag = words + (size_t)a.B * 2 * gang_row_words(a.N, sizeof(T));
     g.state = g.flag + (size_t)a.B * kGangMembers;
     // no word carries a number yet, no member is there, no simulation is marked
@@ -484,7 +502,7 @@ const unsigned long long* gang_state(const unsigned long long* words, int N, int
     return words + (size_t)B * (2 * gang_row_words(N, elem) + kGangMembers);
 }
 
-template hipError_t launch_sim_gang<float>(const float*, const SimArgs&, unsigned long long*, int, hipStream_t);
-template hipError_t launch_sim_gang<double>(const double*, const SimArgs&, unsigned long long*, int, hipStream_t);
+template hipError_t launch_sim_gang<float>(const float*, const SimArgs&, unsigned long long*, int, int, hipStream_t);
+template hipError_t launch_sim_gang<double>(const double*, const SimArgs&, unsigned long long*, int, int, hipStream_t);
 
 }  // namespace bnm

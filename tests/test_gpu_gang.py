@@ -106,20 +106,32 @@ def test_gang_fic_converges(oracle_mod, monkeypatch):
     assert np.abs(g["bold"] - r["bold"]).max() <= 1e-9 * np.abs(r["bold"]).max()
 
 
-@pytest.mark.parametrize("B,gang", [(16, True), (17, False)])
-def test_more_members_than_one_round_holds(B, gang):
-    """FP64 at N = 400 has 13 members a simulation: two of them fit an XCD's 32 CUs,
-    three do not, and such a population runs on one workgroup a simulation."""
-    N = 400
-    print("case: gang rounds B", B, flush=True)
-    cfg = bnm.default_config(nodes=N, n_sims=B, time_steps=60, bold_tr=10, n_vols_remove=0, no_fcd=1,
-                             exc_interhemispheric=0, noise_period_ms=61, max_fic_trials=1, i_sampling_start=10,
-                             i_sampling_end=30, precision=bnm.PREC_F64, fc_precision=bnm.FC_F64)
+@pytest.mark.parametrize("prec,N,B", [(bnm.PREC_F64, 400, 37), (bnm.PREC_F64, 140, 90), (bnm.PREC_F32, 500, 50)], ids=str)
+def test_groups_take_one_simulation_after_the_other(monkeypatch, prec, N, B):
+    """More simulations than groups of resident members, with FIC restarts that make
+    them end at different times, against one workgroup per simulation."""
+    f64 = prec == bnm.PREC_F64
     rng = np.random.default_rng(B)
-    with bnm.Context(cfg) as c:
-        c.set_sc(W.synthetic_sc(N, 0.9, 1))
-        c.set_noise(bnm.make_noise(1, 61 * 20 * N))
-        c.set_empirical(rng.uniform(-0.2, 0.8, bnm.n_pairs(N, False)), rng.uniform(-0.5, 1.0, 40))
-        c.set_params(rng.uniform(0.5, 2.5, B), rng.uniform(0.1, 0.4, (B, N)), rng.uniform(0.1, 0.3, (B, N)))
-        c.run()
-        assert ("gang" in c.tune_log()) == gang, c.tune_log()
+    SC = W.synthetic_sc(N, 0.9, 1)
+    noise = bnm.make_noise(1, 121 * 20 * N)
+    emp = rng.uniform(-0.2, 0.8, bnm.n_pairs(N, False)), rng.uniform(-0.5, 1.0, 40)
+    params = rng.uniform(0.02, 1.5, B), rng.uniform(0.15, 0.25, (B, N)), rng.uniform(0.1, 0.2, (B, N))
+    out = {}
+    for gang in ("1", "0"):
+        print("case: gang groups N", N, "B", B, "gang", gang, flush=True)
+        monkeypatch.setenv("BNM_GANG", gang)
+        cfg = bnm.default_config(nodes=N, n_sims=B, time_steps=120, bold_tr=10, n_vols_remove=0, no_fcd=1,
+                                 exc_interhemispheric=0, noise_period_ms=121, max_fic_trials=2, i_sampling_start=10,
+                                 i_sampling_end=40, precision=prec, fc_precision=bnm.FC_F64)
+        with bnm.Context(cfg) as c:
+            c.set_sc(SC)
+            c.set_noise(noise)
+            c.set_empirical(*emp)
+            c.set_params(*params)
+            c.run()
+            assert c.kernel_name().startswith("gang") == (gang == "1")
+            out[gang] = c.outputs()
+    g, r = out["1"], out["0"]
+    np.testing.assert_array_equal(g["fic_trials"], r["fic_trials"])
+    rel = np.abs(g["bold"] - r["bold"]).max() / np.abs(r["bold"]).max()
+    assert rel <= (1e-9 if f64 else 1e-6)
