@@ -1,5 +1,6 @@
 // math64.hpp -- FP64 exponential, logarithm and reciprocal of the row-blocked and
-// sparse integration kernels, and the Balloon-Windkessel step made of them.
+// multi-workgroup integration kernels, and the row-blocked kernel's
+// Balloon-Windkessel step made of them.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -15,13 +16,12 @@ __device__ __forceinline__ double rcp_f64(double d) {
     return fma(y, fma(e, e, e), y);
 }
 
-// e^y, FP64: y = n ln 2 + f with |f| <= ln 2 / 2, e^f = 1 + f + f^2 Q(f), Q the
+// FP64 e^y by the reduction of Cody and Waite (1980), y = n ln 2 + f with ln 2 in two
+// parts and |f| <= ln 2 / 2: e^y = 2^n (1 + m), m = e^f - 1 = f + f^2 Q(f), Q the
 // degree-9 interpolant of (e^f - 1 - f) / f^2 at Chebyshev nodes (|error| of
-// e^f <= 1.3e-17); about 1 ulp.  y is cut off at 700, where 1 / (1 - e^y) and
-// everything made of it is zero next to any value of the model.
-__device__ __forceinline__ double exp_f64(double y) {
-    y = fmin(y, 700.0);
-    const double n = __builtin_rint(y * kLog2e);
+// e^f <= 1.3e-17).  exp_parts returns m and n.
+__device__ __forceinline__ double exp_parts(double y, double& n) {
+    n = __builtin_rint(y * kLog2e);
     const double f = fma(-n, 0x1.a39ef35793c76p-33, fma(-n, 0x1.62e42fee00000p-1, y));
     const double f2 = f * f, f4 = f2 * f2;
     const double q01 = fma(f, 0x1.5555555555556p-3, 0x1.0000000000001p-1);
@@ -30,20 +30,41 @@ __device__ __forceinline__ double exp_f64(double y) {
     const double q67 = fma(f, 0x1.71de0db21e27fp-19, 0x1.a019b9133a48ap-16);
     const double q89 = fma(f, 0x1.af38a0d2d9620p-26, 0x1.28917e2c43a66p-22);
     const double q = fma(f4, fma(f4, q89, fma(f2, q67, q45)), fma(f2, q23, q01));
-    return __builtin_ldexp(1.0 + fma(f2, q, f), (int)n);
+    return fma(f2, q, f);
 }
 
-// ln v for v > 0, FP64: v = 2^e m with m in [sqrt 1/2, sqrt 2), ln m = 2 s +
-// s^3 W(s^2), s = (m - 1) / (m + 1), W the degree-6 interpolant at Chebyshev
-// nodes (relative error <= 5e-18 of the series); about 1 ulp of ln m.
-__device__ __forceinline__ double log_f64(double v) {
+// 1 - e^y, within 3 ulp for every y, also next to y = 0, where the difference of a
+// rounded e^y from 1 has few digits left: (1 - 2^n) - 2^n m, whose first term is exact
+// for n >= -53 and zero for n = 0.  y is cut off at 700, where 1 / (1 - e^y) and
+// everything made of it is zero next to any value of the model.
+__device__ __forceinline__ double one_minus_exp_f64(double y) {
+    double n;
+    const double m = exp_parts(fmin(y, 700.0), n);
+    const double t = __builtin_ldexp(1.0, (int)n);
+    return fma(-t, m, 1.0 - t);
+}
+
+// e^y, about 1 ulp; y is cut off as above.
+__device__ __forceinline__ double exp_f64(double y) {
+    double n;
+    const double m = exp_parts(fmin(y, 700.0), n);
+    return __builtin_ldexp(1.0 + m, (int)n);
+}
+
+// ln v, FP64, as hi + lo (v > 0 and finite): v = 2^e m with m in [sqrt 1/2, sqrt 2),
+// ln m = 2 s + s^3 W(s^2), s = (m - 1) / (m + 1), W the degree-6 interpolant at
+// Chebyshev nodes (relative error <= 5e-18 of the series).  s is rounded, and so is the
+// m + 1 that it is a quotient by: sl is what s is short of.  hi is the rounded
+// logarithm, lo what that leaves.
+__device__ __forceinline__ double log_parts(double v, double& lo) {
     double m = __builtin_amdgcn_frexp_mant(v);
     int e = __builtin_amdgcn_frexp_exp(v);
     const bool low = m < 0.70710678118654752;
     m = low ? m + m : m;
     e = low ? e - 1 : e;
-    const double d = m - 1.0;
-    const double s = d * rcp_f64(m + 1.0), z = s * s;
+    const double d = m - 1.0, b = m + 1.0;
+    const double rb = rcp_f64(b), s = d * rb, z = s * s;
+    const double sl = fma(-s, m - (b - 1.0), fma(-s, b, d)) * rb;   // (b + (m - (b - 1)) = m + 1)
     double w = 0x1.2b5f68a50d903p-3;
     w = fma(w, z, 0x1.39fdcceb4bb45p-3);
     w = fma(w, z, 0x1.7462b91b8df65p-3);
@@ -51,8 +72,18 @@ __device__ __forceinline__ double log_f64(double v) {
     w = fma(w, z, 0x1.2492492dfd86cp-2);
     w = fma(w, z, 0x1.9999999995273p-2);
     w = fma(w, z, 0x1.5555555555558p-1);
-    const double n = (double)e;
-    return fma(n, 0x1.62e42fee00000p-1, fma(n, 0x1.a39ef35793c76p-33, fma(s * z, w, s + s)));
+    const double n = (double)e, big = n * 0x1.62e42fee00000p-1;   // (exact, and above 2 s or zero)
+    const double h = big + (s + s);
+    const double l = ((big - h) + (s + s)) + fma(n, 0x1.a39ef35793c76p-33, fma(s * z, w, sl + sl));
+    const double hi = h + l;
+    lo = l - (hi - h);
+    return hi;
+}
+
+// v^p for hi + lo = ln v.
+__device__ __forceinline__ double pow_f64(double hi, double lo, double p) {
+    const double y = p * hi, e = exp_f64(y);
+    return fma(e, fma(p, lo, fma(p, hi, -y)), e);
 }
 
 // Balloon-Windkessel step in six parts, so that the row-blocked kernel can run
@@ -123,10 +154,10 @@ template <> struct BWParts<float> : BW<float> {
 };
 
 // FP64: the step of BW<double> with products by reciprocals, exp_f64 and
-// log_f64, and nu^(1/alpha) kept from one step for the next (a step's new nu
+// log_parts, and nu^(1/alpha) kept from one step for the next (a step's new nu
 // is the next one's old nu)
 template <> struct BWParts<double> {
-    double x, f, nu, q, pn, fn, lg, E, rn;
+    double x, f, nu, q, pn, fn, lg, lgl, E, rn;
     __device__ __forceinline__ void reset() { x = 0.0; f = nu = q = pn = 1.0; }
     template <int K>
     __device__ __forceinline__ void part(double SE) {
@@ -136,9 +167,9 @@ template <> struct BWParts<double> {
             fn = fma(C64::model_dt, x, f);
             nu = fma(C64::model_dt * C64::itau, f - pn, nu);
         } else if constexpr (K == 1) {
-            lg = log_f64(nu);
+            lg = log_parts(nu, lgl);
         } else if constexpr (K == 2) {
-            pn = exp_f64(C64::ialpha * lg);
+            pn = pow_f64(lg, lgl, C64::ialpha);
         } else if constexpr (K == 3) {
             E = kLnOneMinRho * rcp_f64(f);
             rn = rcp_f64(nu);

@@ -95,6 +95,10 @@ template <> struct Pool<float> {
     __device__ __forceinline__ void settle() { Sl = S == t ? u - (t - Sp) : 0.0f; }
 };
 
+// FP64, contracted, as exact as the reference's order of operations or more so: the
+// increment of S is formed first, so that S takes one rounding of its own magnitude a
+// substep (three, as a chain of fused operations on S, doubled its error), and 1 - e^y
+// keeps its digits where x is small.
 template <> struct Pool<double> {
     double k0, kS, kO, ac, GJ, aa, bb, nd, g, gm, it;
     double S, r, I;
@@ -126,13 +130,13 @@ template <> struct Pool<double> {
         pre = fma(kO, So, fma(kS, S, k0));
         X0 = fma(aa, pre, -bb);
         A = fma(-gm, S, g);
-        D = fma(-it, S, fma((double)xi, nzs, S));
+        D = fma(-it, S, (double)xi * nzs);
     }
     __device__ __forceinline__ void after(double c, bool last) {
         if (last) I = fma(GJ, c, pre);
         const double x = fma(ac, c, X0);
-        r = x * rcp_f64(1.0 - exp_f64(nd * x));
-        S = fmax(0.0, fmin(fma(r, A, D), 1.0));
+        r = x * rcp_f64(one_minus_exp_f64(nd * x));
+        S = fmax(0.0, fmin(S + fma(r, A, D), 1.0));
     }
     __device__ __forceinline__ void settle() {}
 };

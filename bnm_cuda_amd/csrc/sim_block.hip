@@ -25,10 +25,9 @@
 // ahead into the register that its last draw has left.
 //
 // FP32 is the strict update (hi / lo coefficients as NodeStrict) in own /
-// partner form.  FP64 uses fused multiply-adds, exp_f64 / rcp_f64 and
-// reciprocals of the constants in place of the reference's order of
-// operations; its error against the oracle stays at ~1e-14 (k_sim_ei64, in the
-// reference's order: 1758 cycles).
+// partner form.  FP64 uses fused multiply-adds, the functions of math64.hpp and
+// reciprocals of the constants in place of the reference's order of operations
+// (k_sim_ei64, in that order: 1758 cycles).
 #include <algorithm>
 
 #include "kernels.hpp"
