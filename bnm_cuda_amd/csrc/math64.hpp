@@ -36,7 +36,8 @@ __device__ __forceinline__ double exp_parts(double y, double& n) {
 // 1 - e^y, within 3 ulp for every y, also next to y = 0, where the difference of a
 // rounded e^y from 1 has few digits left: (1 - 2^n) - 2^n m, whose first term is exact
 // for n >= -53 and zero for n = 0.  y is cut off at 700, where 1 / (1 - e^y) and
-// everything made of it is zero next to any value of the model.
+// everything made of it is zero next to any value of the model.  Not for -infinity
+// (NaN) and NaN (cut off too): see Pool<double>::rate().
 __device__ __forceinline__ double one_minus_exp_f64(double y) {
     double n;
     const double m = exp_parts(fmin(y, 700.0), n);
@@ -44,7 +45,7 @@ __device__ __forceinline__ double one_minus_exp_f64(double y) {
     return fma(-t, m, 1.0 - t);
 }
 
-// e^y, about 1 ulp; y is cut off as above.
+// e^y, about 1 ulp; y is cut off as above, and is not -infinity or NaN.
 __device__ __forceinline__ double exp_f64(double y) {
     double n;
     const double m = exp_parts(fmin(y, 700.0), n);
@@ -80,10 +81,13 @@ __device__ __forceinline__ double log_parts(double v, double& lo) {
     return hi;
 }
 
-// v^p for hi + lo = ln v.
-__device__ __forceinline__ double pow_f64(double hi, double lo, double p) {
+// v^p for hi + lo = ln v; NaN unless v is positive and finite (logarithm and
+// exponential have finite values for zero and negative v, and a run that gets there is
+// to end in NaN, as with pow).
+__device__ __forceinline__ double pow_f64(double hi, double lo, double p, double v) {
     const double y = p * hi, e = exp_f64(y);
-    return fma(e, fma(p, lo, fma(p, hi, -y)), e);
+    const double r = fma(e, fma(p, lo, fma(p, hi, -y)), e);
+    return v > 0.0 && v < __builtin_inf() ? r : __builtin_nan("");
 }
 
 // Balloon-Windkessel step in six parts, so that the row-blocked kernel can run
@@ -169,7 +173,7 @@ template <> struct BWParts<double> {
         } else if constexpr (K == 1) {
             lg = log_parts(nu, lgl);
         } else if constexpr (K == 2) {
-            pn = pow_f64(lg, lgl, C64::ialpha);
+            pn = pow_f64(lg, lgl, C64::ialpha, nu);
         } else if constexpr (K == 3) {
             E = kLnOneMinRho * rcp_f64(f);
             rn = rcp_f64(nu);

@@ -68,6 +68,7 @@ template <> struct Pool<float> {
     __device__ __forceinline__ void reset() { S = 0.001f; Sl = NodeStrict::kS0l; }
     __device__ __forceinline__ void set_wIE(bool e) { if (e) NodeStrict::split(-wIE, kOh, kOl); }
     __device__ __forceinline__ double value() const { return (double)S + (double)Sl; }
+    __device__ __forceinline__ double rate() const { return (double)r; }
     __device__ __forceinline__ void before(float xi) {
         constexpr double nzs64 = C64::sigma * C64::sqrt_dt;
         constexpr float nzs = (float)nzs64, nzsl = (float)(nzs64 - (double)nzs);
@@ -124,6 +125,11 @@ template <> struct Pool<double> {
     __device__ __forceinline__ void reset() { S = 0.001; }
     __device__ __forceinline__ void set_wIE(bool e) { if (e) kO = -wIE; }
     __device__ __forceinline__ double value() const { return S; }
+    // r of the last substep, also for an infinite I, where after() leaves NaN (S is 1
+    // either way)
+    __device__ __forceinline__ double rate() const {
+        return fabs(I) < 1e300 ? r : I > 0.0 ? __builtin_inf() : __builtin_nan("");
+    }
     __device__ __forceinline__ void before(float xi) {
         constexpr double nzs = C64::sigma * C64::sqrt_dt;
         const double So = dpp<kXor1>(S);

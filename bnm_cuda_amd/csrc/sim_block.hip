@@ -175,7 +175,7 @@ __global__ __launch_bounds__(MAXT, WAVES) void k_sim_block(const T* __restrict__
             if (vol >= a.n_vols_remove) {
                 ext[0] += p.value();
                 ext[1] += (double)p.I;
-                ext[2] += (double)p.r;
+                ext[2] += p.rate();
             }
             ++vol;
         }

@@ -350,7 +350,7 @@ __device__ __forceinline__ void gang_run(const T* __restrict__ SC, const SimArgs
             if (vol >= a.n_vols_remove) {
                 ext[0] += p.value();
                 ext[1] += (double)p.I;
-                ext[2] += (double)p.r;
+                ext[2] += p.rate();
             }
             ++vol;
         }

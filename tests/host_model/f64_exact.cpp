@@ -4,6 +4,9 @@
 // the host's libm) on the same inputs.
 //
 // "f64_exact functions": largest error in ulp of each function over its ranges.
+// "f64_exact edges": number of cases in which infinite, undefined or far couplings
+// give another S or r than Node<double>, or a Balloon-Windkessel state whose nu is
+// zero, negative, infinite or undefined gives finite BOLD.
 // "f64_exact runs T sims": N = 6 nodes coupled by a random SC, T ms, `sims` parameter
 // sets; prints the rms errors of S_E (every ms) and of BOLD (every 100 ms) of both,
 // over all sets, each set's errors divided by its largest value.
@@ -68,7 +71,7 @@ static double log64(double v) { double lo; const double hi = log_parts(v, lo); r
 static double pow64(double v) {
     double lo;
     const double hi = log_parts(v, lo);
-    return pow_f64(hi, lo, C64::ialpha);
+    return pow_f64(hi, lo, C64::ialpha, v);
 }
 
 static void functions() {
@@ -80,6 +83,44 @@ static void functions() {
     auto dq = [](double x) { return -expm1q(x); };
     ulps("one_minus_exp", -40, 40, false, d, dq);
     ulps("one_minus_exp_small", -30, 0, true, d, dq);
+}
+
+// NaN for NaN, infinity for infinity, otherwise to rel: 1e-13, what cancellation in x
+// leaves, a difference of two values about 125 (one rounding 1.4e-14 each, |x| above 1
+// here)
+static int differ(const char* what, double x, double got, double want, double rel) {
+    const bool same = want != want ? got != got : want == got || std::fabs(got - want) <= rel * std::fabs(want);
+    if (!same) std::fprintf(stderr, "%s(%g) = %g, not %g\n", what, x, got, want);
+    return !same;
+}
+
+static void edges() {
+    const double inf = INFINITY, nan = NAN;
+    int bad = 0;
+    for (double v : std::vector<double>{0.0, -1e-9, -0.5, -1.0, -3e7, inf, nan}) {
+        BWParts<double> b;
+        b.reset();
+        for (int step = 0; step < 3; ++step) {
+            b.nu = step ? b.nu : v;
+            b.part<0>(0.1); b.nu = step ? b.nu : v;
+            b.part<1>(0.1); b.part<2>(0.1); b.part<3>(0.1); b.part<4>(0.1); b.part<5>(0.1);
+        }
+        const double B = b.bold(C64::k1, C64::k2, C64::k3);
+        if (B == B) { std::fprintf(stderr, "BOLD for nu = %g: %g\n", v, B); ++bad; }
+    }
+    for (double v : std::vector<double>{0.0, 1.0, 1e4, 1e9, 1e30, inf, -1e3, -1e9, -inf, nan}) {
+        double SE = 0.001, SI = 0.001, IE, II, rE, rI;
+        Node<double>::step(v, 1.0, 0.2, 0.2, 1.0, 0.125, 0.125, SE, SI, IE, II, rE, rI);
+        Pool<double> e;
+        e.init(0, 1.0, 0.2, 0.2, 1.0);
+        partner(0.001);
+        e.before(0.125f);
+        e.after(v, true);
+        // (for a far negative x the rate is zero beside anything: below 1e-200)
+        bad += differ("S_E", v, e.S, SE, 1e-13) +
+               differ("r_E", v, std::fabs(e.rate()) < 1e-200 ? 0.0 : e.rate(), std::fabs(rE) < 1e-200 ? 0.0 : rE, 1e-13);
+    }
+    std::printf("edges %d\n", bad);
 }
 
 struct Exact {
@@ -194,6 +235,7 @@ static void runs(int T, int sims) {
 
 int main(int argc, char** argv) {
     if (argc == 2 && !std::strcmp(argv[1], "functions")) functions();
+    else if (argc == 2 && !std::strcmp(argv[1], "edges")) edges();
     else if (argc == 4) runs(std::atoi(argv[2]), std::atoi(argv[3]));
     else return 2;
     return 0;

@@ -44,6 +44,12 @@ def test_functions_within_ulps(exe):
         assert v[k] <= b, k
 
 
+def test_edge_values(exe):
+    """Infinite, undefined and far values end as they do in the reference's order (NaN
+    BOLD, hence the largest cost; an infinite rate), not in other finite values."""
+    assert _values(exe, "edges") == dict(edges=0)
+
+
 def test_runs_no_less_exact_than_the_reference_order(exe):
     v = _values(exe, "runs", "3000", "8")
     assert v["S_kernels"] <= 1.25 * v["S_reference"]
