@@ -31,7 +31,7 @@ EXPORTS = (
     "bnm_window_bounds", "bnm_regional_params", "bnm_analytical_fic", "bnm_make_noise", "bnm_make_noise_chunked", "bnm_sparse_layout", "bnm_run_simulations", "bnm_run_simulations_noalloc", "bnm_ctx_create",
     "bnm_ctx_destroy", "bnm_ctx_set_sc", "bnm_ctx_set_noise", "bnm_ctx_set_empirical",
     "bnm_ctx_set_params", "bnm_ctx_run", "bnm_ctx_set_bold", "bnm_ctx_analyze", "bnm_ctx_get_hemi_fcd", "bnm_ctx_get_outputs", "bnm_ctx_get_ext", "bnm_ctx_timings",
-    "bnm_ctx_kernel_name", "bnm_ctx_tune_log", "bnm_multi_create", "bnm_multi_run",
+    "bnm_ctx_kernel_name", "bnm_ctx_taken_over", "bnm_ctx_tune_log", "bnm_multi_create", "bnm_multi_run",
     "bnm_multi_last_ms", "bnm_multi_plan", "bnm_multi_destroy", "bnm_cmaes_create", "bnm_cmaes_destroy",
     "bnm_cmaes_ask", "bnm_cmaes_tell", "bnm_cmaes_best", "bnm_cmaes_sigma", "bnm_cmaes_strategy", "bnm_cmaes_iteration", "bnm_cmaes_ask_pool", "bnm_cmaes_select",
     "bnm_mlp_create", "bnm_mlp_destroy", "bnm_mlp_num_params", "bnm_mlp_get_params",
@@ -109,6 +109,7 @@ def lib():
     L.bnm_ctx_timings.argtypes = [vp, pd, C.c_int]
     L.bnm_ctx_kernel_name.argtypes = [vp]
     L.bnm_ctx_kernel_name.restype = C.c_char_p
+    L.bnm_ctx_taken_over.argtypes = [vp]
     L.bnm_ctx_tune_log.argtypes = [vp]
     L.bnm_ctx_tune_log.restype = C.c_char_p
     L.bnm_multi_create.argtypes = [C.POINTER(vp), C.c_int, pi]
@@ -341,6 +342,11 @@ class Context:
 
     def kernel_name(self):
         return lib().bnm_ctx_kernel_name(self.h).decode()
+
+    def taken_over(self):
+        """Simulations of the last run whose workgroups did not meet and that one
+        workgroup each ran instead (same results)."""
+        return _chk(lib().bnm_ctx_taken_over(self.h))
 
     def tune_log(self):
         return lib().bnm_ctx_tune_log(self.h).decode()

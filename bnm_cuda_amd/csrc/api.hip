@@ -152,12 +152,12 @@ struct bnm_ctx {
     int autotune = 1, tune_ms = 300;
     Variant variant{0, 4, 1, 0};
     // the best variant with one workgroup per simulation: what a graph of several
-    // contexts runs (its branches fill the CUs), and what runs the simulations
-    // whose workgroups did not find each other
+    // contexts runs (its branches fill the CUs)
     Variant solo{0, 4, 1, 0};
     double solo_ms_per_sim_ms = -1;
     unsigned long long* gang = nullptr;   // exchange words of kind 10
-    int gang_mode = -1, gang_polls = kGangStartPolls;
+    int gang_mode = -1, gang_polls = kGangStartPolls, gang_mark = 0;
+    bool gang_ran = false;   // the last run was kind 10's
     int cus = 256;
     hipGraphExec_t graph_exec = nullptr;
     bool have_sc = false, have_noise = false, have_emp = false, have_params = false;
@@ -403,7 +403,10 @@ static int ctx_alloc(bnm_ctx* x) {
     int r;
     if ((r = cdalloc(x, &x->SC64, N * N))) return r;
     if ((r = cdalloc(x, &x->SC32, N * N))) return r;
-    if ((r = cdalloc(x, &x->SCt64, N * N))) return r;
+    // (kSCtPad zero rows after the N rows where the multi-workgroup kernel may read them)
+    const size_t pad64 = !x->arena && x->f64 && gang_shape(x->N, 8).ok ? kSCtPad : 0;
+    if ((r = cdalloc(x, &x->SCt64, (N + pad64) * N))) return r;
+    if (pad64) HIPCHK(hipMemset(x->SCt64, 0, (N + pad64) * N * sizeof(double)));
     // kSCtPad zero rows after the N rows: the hybrid kernel's padded k-ranges
     // read them without bounds checks
     if ((r = cdalloc(x, &x->SCt32, (N + kSCtPad) * N))) return r;
@@ -620,10 +623,11 @@ static bnm_ctx* ctx_create(const bnm_config* cfg, int* status, unsigned char* ar
     x->sparse_mode = env_int("BNM_SPARSE_STRICT", 1) ? 64 : 0;
     // BNM_GANG: 1 pins the kernel with several workgroups per simulation where it
     // applies, 0 leaves it out; BNM_GANG_POLLS: how long a workgroup waits for
-    // the others of its simulation (-1: not at all, every simulation then runs on
-    // one workgroup)
+    // the others of its simulation (-1: one look); BNM_GANG_MARK=n: every n-th
+    // simulation runs on one workgroup, as if its workgroups had not met
     x->gang_mode = env_int("BNM_GANG", -1);
     x->gang_polls = env_int("BNM_GANG_POLLS", kGangStartPolls);
+    x->gang_mark = env_int("BNM_GANG_MARK", 0);
     x->hyb_ks = env_int("BNM_HYB_KS", 0);
     {
         int dev = 0, v = 0;
@@ -899,14 +903,9 @@ static hipError_t launch_variant(bnm_ctx* x, const Variant& v, const SimArgs& a,
             return launch_sim_sparse(x->SPw[v.ls - 1], x->SPd[v.ls - 1], a, x->sp_P[v.ls - 1], v.ls, (v.mode & 64) != 0,
                                      x->lds_max, st);
         case 9: return x->f64 ? launch_sim_block<double>(x->SC64, a, st) : launch_sim_block<float>(x->SC32, a, st);
-        case 10: {
-            const hipError_t e = x->f64 ? launch_sim_gang<double>(x->SC64, a, x->gang, x->gang_polls, x->cus, st)
-                                        : launch_sim_gang<float>(x->SC32, a, x->gang, x->gang_polls, x->cus, st);
-            if (e != hipSuccess) return e;
-            SimArgs b = a;
-            b.only = gang_state(x->gang, x->N, x->B, x->f64 ? 8 : 4);
-            return launch_variant(x, x->solo, b, st);
-        }
+        case 10:
+            return x->f64 ? launch_sim_gang<double>(x->SC64, x->SCt64, a, x->gang, x->gang_polls, x->gang_mark, x->cus, st)
+                          : launch_sim_gang<float>(x->SC32, x->SCt32, a, x->gang, x->gang_polls, x->gang_mark, x->cus, st);
         default:
             return x->f64 ? launch_sim_plain<double>(x->SC64, a, st)
                           : launch_sim_plain<float>(x->SC32, a, st);
@@ -1300,6 +1299,7 @@ int bnm_ctx_run(bnm_ctx* x) {
         HIPCHK(hipStreamSynchronize(x->st));
         for (int i = 0; i < 6; ++i) x->timings[i] = -1;
         x->have_bold = true;
+        x->gang_ran = x->variant.kind == 10;
         return BNM_OK;
     }
     if (x->cfg.use_graph) {
@@ -1323,6 +1323,7 @@ int bnm_ctx_run(bnm_ctx* x) {
         for (int i = 0; i < 5; ++i) x->timings[i] = -1;
         x->timings[5] = ms;
         x->have_bold = true;
+        x->gang_ran = x->variant.kind == 10;
         return BNM_OK;
     }
     r = enqueue_run(x, x->st, true);
@@ -1338,6 +1339,7 @@ int bnm_ctx_run(bnm_ctx* x) {
     HIPCHK(hipEventElapsedTime(&ms, x->ev[0], x->ev[5]));
     x->timings[5] = ms;
     x->have_bold = true;
+    x->gang_ran = x->variant.kind == 10;
     return BNM_OK;
 }
 
@@ -1568,6 +1570,7 @@ int bnm_multi_run(bnm_multi* m) {
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, m->t0, m->t1));
     m->ms = ms;
+    for (bnm_ctx* c : m->ctxs) c->gang_ran = false;
     return BNM_OK;
 }
 
@@ -1585,6 +1588,17 @@ void bnm_multi_destroy(bnm_multi* m) {
     for (hipEvent_t e : m->joins)
         if (e) (void)hipEventDestroy(e);
     delete m;
+}
+
+int bnm_ctx_taken_over(bnm_ctx* x) {
+    if (!x) return fail(BNM_E_ARG, "null context");
+    if (!x->gang_ran) return 0;
+    std::vector<unsigned long long> state(x->B);
+    HIPCHK(hipMemcpy(state.data(), gang_state(x->gang, x->N, x->B, x->f64 ? 8 : 4), state.size() * 8,
+                     hipMemcpyDeviceToHost));
+    int n = 0;
+    for (unsigned long long v : state) n += (int)(v >> 63);
+    return n;
 }
 
 const char* bnm_ctx_tune_log(bnm_ctx* x) { return x ? x->tune_log.c_str() : ""; }

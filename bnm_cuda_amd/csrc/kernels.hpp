@@ -95,8 +95,9 @@ hipError_t launch_sim_block(const T* SC, const SimArgs& a, hipStream_t st);
 // multi-workgroup kernel (sim_gang.hip): FP32 N of 257 to 512, FP64 129 to 512;
 // `words` holds gang_words() 64-bit words and is cleared by the launch.  A
 // simulation whose workgroups did not find each other is marked in
-// gang_state() (top bit) and has no results: a launch of another kernel with
-// SimArgs::only = gang_state() runs those.
+// gang_state() (top bit) and run by a second kernel of the launch on one
+// workgroup, with the same results.  mark > 0: every mark-th simulation is
+// marked from the start.
 constexpr int kGangMembers = 16, kGangThreads = 512, kGangStartPolls = 1 << 16;
 struct GangArgs {
     int C;                         // workgroups per simulation
@@ -115,8 +116,8 @@ GangShape gang_shape(int N, size_t elem);
 size_t gang_words(int N, int B, size_t elem);
 const unsigned long long* gang_state(const unsigned long long* words, int N, int B, size_t elem);
 template <class T>
-hipError_t launch_sim_gang(const T* SC, const SimArgs& a, unsigned long long* words, int start_polls, int cus,
-                           hipStream_t st);
+hipError_t launch_sim_gang(const T* SC, const T* SCt, const SimArgs& a, unsigned long long* words, int start_polls,
+                           int mark, int cus, hipStream_t st);
 template <class R>
 hipError_t launch_sim_stream(const R* SCt, const SimArgs& a, int KS, hipStream_t st);
 

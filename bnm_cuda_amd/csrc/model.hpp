@@ -410,7 +410,6 @@ struct SimArgs {
     int* fic_failed;          // [B]
     int* fic_trials;          // [B]
     double bw_k1, bw_k2, bw_k3;   // BOLD weights (C64::k1..k3 or k1_F..k3_F)
-    const unsigned long long* only;   // null, or [B]: only the simulations whose top bit is set run
 };
 
 }  // namespace bnm

@@ -25,8 +25,9 @@
 // Waiting: members start when all are there and on one XCD.  A member that waits
 // in vain (GangArgs::start_polls, another kernel holds the CUs) marks the
 // simulation, every member of a marked simulation ends, and the launch that
-// follows in the stream (SimArgs::only) runs the marked simulations on one
-// workgroup each.  From then on all members are resident, and the polls in the
+// follows in the stream (k_sim_gang_alone) runs the marked simulations on one
+// workgroup each, with the members' arithmetic: a simulation's results do not depend on
+// whether its members met.  From then on all members are resident, and the polls in the
 // time loop end when the others get there; they have a bound too (kLoopPolls),
 // with the same consequence.  A group of members runs one simulation after the other,
 // as many groups as have a CU for each member: members of a second round of
@@ -439,6 +440,155 @@ __global__ __launch_bounds__(kGangThreads) void k_sim_gang(const T* __restrict__
     }
 }
 
+// The simulations that are marked, one workgroup each, with the bits of gang_run: a
+// node's sum is that of 16 slices of KC values, each an FMA chain in order of k, added
+// in gang_sum's tree.  That is, with s_q the sum of slice q, (T_0 + T_2) + (T_1 + T_3),
+// R = 4: T_i = (s_i + s_15-i) + (s_i+8 + s_7-i), R = 2: (s_i + s_i+8) + (s_i+4 + s_i+12).
+// A lane sums slices of one node, with SC streamed column by column from L2: KS waves a
+// node, one T_i each, or two.  Then a lane steps one pool.  Bound by that stream: N = 400,
+// FP32, 11 us a substep, FP64 21.
+template <class T, int R, int KC>
+__global__ __launch_bounds__(1024) void k_sim_gang_alone(const T* __restrict__ SCt, SimArgs a, const u64* __restrict__ state,
+                                                         int KS) {
+    constexpr bool F64 = sizeof(T) == 8;
+    const int sim = blockIdx.x;
+    if (!(state[sim] & kGangAbort)) return;
+    const int N = a.N, NW = (N + 63) / 64, tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = wave % NW, ks = wave / NW;
+    const int col = nw * 64 + lane, colc = min(col, N - 1);          // the node that this lane sums for
+    const int pop = tid & 1, j = tid >> 1, jc = min(j, N - 1);        // the pool that it steps
+    const bool comp = j < N, writer = comp && pop == 0, steps = wave * 32 < N;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    constexpr int ldS = 16 * KC;                    // (S_E past the last node is 0, and so is SCt)
+    T* Sb = reinterpret_cast<T*>(smem_raw);         // [2][ldS]
+    T* part = Sb + 2 * ldS;                         // [KS][64 NW]
+    const __amdgpu_buffer_rsrc_t scr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(SCt), (short)0, (N + (int)kSCtPad) * N * (int)sizeof(T), 0x00020000);
+    const int voff = colc * (int)sizeof(T);
+    auto column = [&](int k) __attribute__((always_inline)) {             // SC[the lane's node][k]
+        const int so = k * N * (int)sizeof(T);
+        if constexpr (F64) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(scr, voff, so, 0);
+            return __longlong_as_double(((long long)v[1] << 32) | v[0]);
+        } else {
+            return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(scr, voff, so, 0));
+        }
+    };
+    auto four = [&](const T* S, int i) __attribute__((always_inline)) {   // T_i
+        const int sl[4] = {i, R == 4 ? 15 - i : i + 8, R == 4 ? i + 8 : i + 4, R == 4 ? 7 - i : i + 12};
+        constexpr int U = 4;                        // (x 4 loads on the way together)
+        T s[4] = {T(0), T(0), T(0), T(0)};
+        auto batch = [&](auto n, int m0) __attribute__((always_inline)) {
+            constexpr int M = decltype(n)::value;
+            T w[M][4];
+#pragma unroll
+            for (int u = 0; u < M; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) w[u][q] = column(sl[q] * KC + m0 + u);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < M; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s[q] = fma(w[u][q], S[sl[q] * KC + m0 + u], s[q]);
+        };
+#pragma unroll 1
+        for (int m0 = 0; m0 + U <= KC; m0 += U) batch(std::integral_constant<int, U>{}, m0);
+        if constexpr (KC % U != 0) batch(std::integral_constant<int, KC % U>{}, KC / U * U);
+        return (s[0] + s[1]) + (s[2] + s[3]);
+    };
+    for (int i = tid; i < 2 * ldS; i += blockDim.x) Sb[i] = i % ldS < N ? T(0.001) : T(0);
+    const size_t o = (size_t)sim * N + jc;
+    Pool<T> p;
+    p.init(pop, a.G[sim], a.wEE[o], a.wEI[o], a.wIE_in[o]);
+    double delta = a.init_delta;
+    typename std::conditional<F64, BW<double>, BWParts<float>>::type bw;
+    bw.reset();
+    double mI = 0, ext[3] = {0, 0, 0};
+    int ts = 0, vol = 0, trial = 0;
+    bool adjusting = a.adjust_fic != 0, failed = false;
+    const unsigned dur = (unsigned)(a.i_end - a.i_start + 1);
+    const int P = (int)a.noise_period;
+    auto draw = [&](int ms, int s) { return a.noise[(((size_t)ms * 10 + s) * N + jc) * 2 + pop]; };
+    p.before(draw(0, 0));
+    __syncthreads();
+    while (ts <= a.time_steps) {
+        const int ms = ts % P, ms1 = ms + 1 == P ? 0 : ms + 1;
+#pragma unroll 1
+        for (int s = 0; s < 10; ++s) {
+            const T* S = Sb + (s & 1) * ldS;
+            const float drawn = s < 9 ? draw(ms, s + 1) : draw(ms1, 0);
+            part[ks * 64 * NW + col] = KS == 4 ? four(S, ks) : four(S, ks) + four(S, ks + 2);
+            __syncthreads();
+            if (steps) {
+                const T* c = part + jc;
+                const int ld = 64 * NW;
+                p.after(KS == 4 ? (c[0] + c[2 * ld]) + (c[ld] + c[3 * ld]) : c[0] + c[ld], s == 9);
+                if (writer) Sb[((s + 1) & 1) * ldS + j] = p.S;
+                p.settle();
+                p.before(drawn);
+            }
+            __syncthreads();
+        }
+        if constexpr (F64) {
+            bw.step(p.S);
+        } else {
+            bw.template part<0>(p.S);
+            bw.template part<1>(p.S);
+            bw.template part<2>(p.S);
+            bw.template part<3>(p.S);
+            bw.template part<4>(p.S);
+            bw.template part<5>(p.S);
+        }
+        if (ts % a.bold_tr == 0) {
+            if (writer)
+                reinterpret_cast<T*>(a.bold)[((size_t)sim * a.output_ts + vol) * N + j] =
+                    (T)bw.bold(a.bw_k1, a.bw_k2, a.bw_k3);
+            if (vol >= a.n_vols_remove) {
+                ext[0] += p.value();
+                ext[1] += (double)p.I;
+                ext[2] += p.rate();
+            }
+            ++vol;
+        }
+        ++ts;
+        if (adjusting) {
+            if (ts >= a.i_start && ts <= a.i_end) mI += (double)p.I;
+            if (ts == a.i_end) {
+                const bool out = writer && fic_decide<double>(mI, dur, trial, a.max_fic_trials, p.wIE, delta);
+                p.set_wIE(pop == 0);
+                if (!__syncthreads_or(out)) {
+                    adjusting = false;
+                } else if (trial < a.max_fic_trials) {
+                    p.reset();
+                    bw.reset();
+                    mI = 0;
+                    ext[0] = ext[1] = ext[2] = 0;
+                    if (writer) Sb[j] = p.S;
+                    ts = 0; vol = 0; ++trial;
+                    p.before(draw(0, 0));
+                    __syncthreads();
+                } else {
+                    failed = true; adjusting = false;
+                }
+            }
+        }
+    }
+    if (comp) {
+        if (pop == 0) a.wIE_out[o] = p.wIE;
+        const int n = vol - a.n_vols_remove;
+        for (int i = 0; i < 3; ++i) a.ext[((size_t)sim * 6 + 3 * pop + i) * N + j] = n > 0 ? ext[i] / n : 0.0;
+    }
+    if (tid == 0) {
+        a.fic_failed[sim] = failed ? 1 : 0;
+        a.fic_trials[sim] = trial;
+    }
+}
+
+// marks every n-th simulation before any member looks
+__global__ void k_gang_mark(u64* state, int B, int n) {
+    for (int i = threadIdx.x * n; i < B; i += blockDim.x * n) state[i] = kGangAbort;
+}
+
 // FP32: N of 257 to 512, R = 4 (64 nodes a member).  FP64: 129 to 256 with R = 4,
 // to 512 with R = 2 (32 nodes a member: R x KC doubles are the same VGPRs).
 static const int kGangKC[] = {10, 13, 16, 20, 25, 28, 32};
@@ -466,14 +616,17 @@ size_t gang_words(int N, int B, size_t elem) {
 }
 
 template <class T, int R, int KC>
-static void launch_gang(const T* SC, const SimArgs& a, const GangArgs& g, const GangShape& s, hipStream_t st) {
+static void launch_gang(const T* SC, const T* SCt, const SimArgs& a, const GangArgs& g, const GangShape& s, hipStream_t st) {
     hipLaunchKernelGGL((k_sim_gang<T, R, KC>), dim3(8 * s.C * g.groups), dim3(kGangThreads), s.smem, st, SC, a,
                        g, s.SS);
+    const int NW = (a.N + 63) / 64, KS = NW <= 4 ? 4 : 2;
+    const size_t smem = (2 * 16 * KC + KS * 64 * (size_t)NW) * sizeof(T);
+    hipLaunchKernelGGL((k_sim_gang_alone<T, R, KC>), dim3(a.B), dim3(KS * 64 * NW), smem, st, SCt, a, g.state, KS);
 }
 
 template <class T>
-hipError_t launch_sim_gang(const T* SC, const SimArgs& a, unsigned long long* words, int start_polls, int cus,
-                           hipStream_t st) {
+hipError_t launch_sim_gang(const T* SC, const T* SCt, const SimArgs& a, unsigned long long* words, int start_polls,
+                           int mark, int cus, hipStream_t st) {
     const GangShape s = gang_shape(a.N, sizeof(T));
     if (!s.ok) return hipErrorInvalidValue;
     GangArgs g{};
@@ -486,14 +639,15 @@ hipError_t launch_sim_gang(const T* SC, const SimArgs& a, unsigned long long* wo
     // no word carries a number yet, no member is there, no simulation is marked
     hipError_t e = launch_fill_i32(reinterpret_cast<int*>(words), (long long)gang_words(a.N, a.B, sizeof(T)) * 2, 0, st);
     if (e != hipSuccess) return e;
+    if (mark > 0) hipLaunchKernelGGL(k_gang_mark, dim3(1), dim3(256), 0, st, g.state, a.B, mark);
     switch (s.KC) {
-        case 10: if constexpr (sizeof(T) == 8) launch_gang<T, 4, 10>(SC, a, g, s, st); break;
-        case 13: if constexpr (sizeof(T) == 8) launch_gang<T, 4, 13>(SC, a, g, s, st); break;
-        case 16: if constexpr (sizeof(T) == 8) launch_gang<T, 4, 16>(SC, a, g, s, st); break;
-        case 20: launch_gang<T, sizeof(T) == 4 ? 4 : 2, 20>(SC, a, g, s, st); break;
-        case 25: launch_gang<T, sizeof(T) == 4 ? 4 : 2, 25>(SC, a, g, s, st); break;
-        case 28: launch_gang<T, sizeof(T) == 4 ? 4 : 2, 28>(SC, a, g, s, st); break;
-        default: launch_gang<T, sizeof(T) == 4 ? 4 : 2, 32>(SC, a, g, s, st); break;
+        case 10: if constexpr (sizeof(T) == 8) launch_gang<T, 4, 10>(SC, SCt, a, g, s, st); break;
+        case 13: if constexpr (sizeof(T) == 8) launch_gang<T, 4, 13>(SC, SCt, a, g, s, st); break;
+        case 16: if constexpr (sizeof(T) == 8) launch_gang<T, 4, 16>(SC, SCt, a, g, s, st); break;
+        case 20: launch_gang<T, sizeof(T) == 4 ? 4 : 2, 20>(SC, SCt, a, g, s, st); break;
+        case 25: launch_gang<T, sizeof(T) == 4 ? 4 : 2, 25>(SC, SCt, a, g, s, st); break;
+        case 28: launch_gang<T, sizeof(T) == 4 ? 4 : 2, 28>(SC, SCt, a, g, s, st); break;
+        default: launch_gang<T, sizeof(T) == 4 ? 4 : 2, 32>(SC, SCt, a, g, s, st); break;
     }
     return hipGetLastError();
 }
@@ -502,7 +656,9 @@ const unsigned long long* gang_state(const unsigned long long* words, int N, int
     return words + (size_t)B * (2 * gang_row_words(N, elem) + kGangMembers);
 }
 
-template hipError_t launch_sim_gang<float>(const float*, const SimArgs&, unsigned long long*, int, int, hipStream_t);
-template hipError_t launch_sim_gang<double>(const double*, const SimArgs&, unsigned long long*, int, int, hipStream_t);
+template hipError_t launch_sim_gang<float>(const float*, const float*, const SimArgs&, unsigned long long*, int, int, int,
+                                           hipStream_t);
+template hipError_t launch_sim_gang<double>(const double*, const double*, const SimArgs&, unsigned long long*, int, int,
+                                            int, hipStream_t);
 
 }  // namespace bnm

@@ -962,7 +962,6 @@ __global__ __launch_bounds__(MAXT) void k_sim_hyb64(const double* __restrict__ S
     constexpr int CH = 8;
     static_assert(RR % CH == 0, "register part must be whole chunks");
     const int sim = blockIdx.x;
-    if (a.only && !(a.only[sim] >> 63)) return;
     const int N = a.N;
     const int T = blockDim.x;
     const int tid = threadIdx.x;
@@ -1112,7 +1111,6 @@ __global__ __launch_bounds__(1024) void k_sim_split_g(const R* __restrict__ SCt,
     constexpr int VW = sizeof(V) / sizeof(R);
     constexpr int CH = 16;  // k per chunk
     const int sim = blockIdx.x;
-    if (a.only && !(a.only[sim] >> 63)) return;
     const int N = a.N;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int nw = wave % NW, ks = wave / NW;
@@ -1243,7 +1241,6 @@ __global__ __launch_bounds__(MAXT) void k_sim_hyb(const float* __restrict__ SCc,
     constexpr int CH = 16;
     static_assert(RR % CH == 0, "register part must be whole chunks");
     const int sim = blockIdx.x;
-    if (a.only && !(a.only[sim] >> 63)) return;
     const int N = a.N;
     const int T = blockDim.x;
     const int tid = threadIdx.x;
@@ -1498,7 +1495,6 @@ __global__ __launch_bounds__(MAXT) void k_sim_sparse(const R* __restrict__ Wsp, 
     constexpr int DW = (RW + LLMAX) / 4;
     constexpr int GN = 64 / LS;   // nodes per wave
     const int sim = blockIdx.x;
-    if (a.only && !(a.only[sim] >> 63)) return;
     const int N = a.N;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sl = lane / GN;                      // the lane's slice of the row

@@ -268,6 +268,11 @@ int bnm_ctx_timings(bnm_ctx* ctx, double* ms, int n);
  * shape (for reports). */
 const char* bnm_ctx_kernel_name(bnm_ctx* ctx);
 
+/* Number of simulations of the last bnm_ctx_run whose workgroups did not meet
+ * (another kernel held the CUs) and that ran on one workgroup each, with the
+ * same results; 0 for kernels with one workgroup per simulation, < 0 on error. */
+int bnm_ctx_taken_over(bnm_ctx* ctx);
+
 /* Integration variants the autotuner timed and their times (empty when it
  * did not run). */
 const char* bnm_ctx_tune_log(bnm_ctx* ctx);
