@@ -624,7 +624,8 @@ static bnm_ctx* ctx_create(const bnm_config* cfg, int* status, unsigned char* ar
     // BNM_GANG: 1 pins the kernel with several workgroups per simulation where it
     // applies, 0 leaves it out; BNM_GANG_POLLS: how long a workgroup waits for
     // the others of its simulation (-1: one look); BNM_GANG_MARK=n: every n-th
-    // simulation runs on one workgroup, as if its workgroups had not met
+    // simulation runs on one workgroup, as if its workgroups had not met, n < 0:
+    // the last workgroup of each group does not come
     x->gang_mode = env_int("BNM_GANG", -1);
     x->gang_polls = env_int("BNM_GANG_POLLS", kGangStartPolls);
     x->gang_mark = env_int("BNM_GANG_MARK", 0);

@@ -97,15 +97,18 @@ hipError_t launch_sim_block(const T* SC, const SimArgs& a, hipStream_t st);
 // simulation whose workgroups did not find each other is marked in
 // gang_state() (top bit) and run by a second kernel of the launch on one
 // workgroup, with the same results.  mark > 0: every mark-th simulation is
-// marked from the start.
-constexpr int kGangMembers = 16, kGangThreads = 512, kGangStartPolls = 1 << 16;
+// marked from the start; mark < 0: the last workgroup of every group stays
+// away.
+constexpr int kGangMembers = 16, kGangThreads = 512, kGangStartPolls = 1 << 22;
 struct GangArgs {
     int C;                         // workgroups per simulation
     int groups;                    // of C workgroups on each XCD
-    int start_polls;               // polls of ~0.5 us that a workgroup waits for the others
+    int present;                   // members of a group that come, C
+    int start_polls;               // polls of ~0.4 us that a workgroup waits for the others
     unsigned long long* xch;       // [B][2][words of a row]
     unsigned long long* flag;      // [B][kGangMembers]
     unsigned long long* state;     // [B] members present, top bit: given up
+    unsigned long long* gave_up;   // a member has waited in vain
 };
 struct GangShape {
     int R, KC, SS, C;

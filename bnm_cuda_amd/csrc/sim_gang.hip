@@ -23,8 +23,12 @@
 // wait for its noise from HBM first.
 //
 // Waiting: members start when all are there and on one XCD.  A member that waits
-// in vain (GangArgs::start_polls, another kernel holds the CUs) marks the
-// simulation, every member of a marked simulation ends, and the launch that
+// in vain (GangArgs::start_polls, 1.5 s: another kernel holds the CUs) marks the
+// simulation, and tells the rest of the launch, whose members then wait no more: those
+// that do not find all the others there mark at once, so a launch waits once.  It waits
+// that long because the CUs mostly come free: two contexts of 32 simulations of N = 400,
+// FP32, each 0.155 s by itself, run at the same time take 0.31 s (0.60 s with a wait of
+// 33 ms for each simulation).  Every member of a marked simulation ends, and the launch that
 // follows in the stream (k_sim_gang_alone) runs the marked simulations on one
 // workgroup each, with the members' arithmetic: a simulation's results do not depend on
 // whether its members met.  From then on all members are resident, and the polls in the
@@ -142,7 +146,9 @@ __device__ __forceinline__ void gang_run(const T* __restrict__ SC, const SimArgs
             if (v & kGangAbort) { d = 1; break; }
             const bool all = (int)(v & 255) >= C;
             if (all && (int)((v >> sh) & 31) == C) break;
-            if ((all || n >= ga.start_polls) &&
+            if (!all && n >= ga.start_polls)
+                __hip_atomic_store(ga.gave_up, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if ((all || xload(ga.gave_up)) &&
                 __hip_atomic_compare_exchange_strong(state, &v, v | kGangAbort, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT)) {
                 d = 1;
@@ -434,6 +440,7 @@ __device__ __forceinline__ void gang_run(const T* __restrict__ SC, const SimArgs
 template <class T, int R, int KC>
 __global__ __launch_bounds__(kGangThreads) void k_sim_gang(const T* __restrict__ SC, SimArgs a, GangArgs ga, int SS) {
     const int member = (blockIdx.x >> 3) % ga.C;
+    if (member >= ga.present) return;
     for (int sim = (blockIdx.x >> 3) / ga.C * 8 + (blockIdx.x & 7); sim < a.B; sim += 8 * ga.groups) {
         gang_run<T, R, KC>(SC, a, ga, SS, member, sim);
         __syncthreads();
@@ -612,7 +619,7 @@ GangShape gang_shape(int N, size_t elem) {
 static size_t gang_row_words(int N, size_t elem) { return elem == 4 ? ((size_t)N + 1) / 2 * 2 : 2 * (size_t)N; }
 
 size_t gang_words(int N, int B, size_t elem) {
-    return (size_t)B * (gang_row_words(N, elem) * 2 + kGangMembers + 1);
+    return (size_t)B * (gang_row_words(N, elem) * 2 + kGangMembers + 1) + 1;
 }
 
 template <class T, int R, int KC>
@@ -636,6 +643,8 @@ hipError_t launch_sim_gang(const T* SC, const T* SCt, const SimArgs& a, unsigned
     g.groups = std::max(1, std::min((a.B + 7) / 8, cus / 8 / s.C));   // per XCD
     g.flag = words + (size_t)a.B * 2 * gang_row_words(a.N, sizeof(T));
     g.state = g.flag + (size_t)a.B * kGangMembers;
+    g.gave_up = g.state + a.B;
+    g.present = mark < 0 ? s.C - 1 : s.C;
     // no word carries a number yet, no member is there, no simulation is marked
     hipError_t e = launch_fill_i32(reinterpret_cast<int*>(words), (long long)gang_words(a.N, a.B, sizeof(T)) * 2, 0, st);
     if (e != hipSuccess) return e;

@@ -57,3 +57,34 @@ def test_same_bits_in_a_graph(monkeypatch):
     assert (a[0], b[0]) == (0, 2)
     for k in KEYS:
         np.testing.assert_array_equal(a[1][k], b[1][k], err_msg=k)
+
+
+def test_a_launch_waits_once(monkeypatch):
+    """A workgroup that never comes is waited for once a launch, not once a simulation:
+    with 1024 simulations on 32 groups, 32 simulations a group, a longer patience costs
+    its own length, not 32 times that.  (A poll takes between 0.3 and 3 us, so 40000
+    polls 12 to 120 ms, and 31 more waits 0.37 s at least.)"""
+    N, B, T = 500, 1024, 2
+    monkeypatch.setenv("BNM_GANG", "1")
+    took = []
+    for mark, polls in ((1, 0), (-1, 40000)):
+        print("case: gang waits, mark", mark, "polls", polls, flush=True)
+        monkeypatch.setenv("BNM_GANG_MARK", str(mark))
+        monkeypatch.setenv("BNM_GANG_POLLS", str(polls))
+        cfg = bnm.default_config(nodes=N, n_sims=B, time_steps=T, bold_tr=1, n_vols_remove=0, no_fcd=1,
+                                 exc_interhemispheric=0, noise_period_ms=T + 1, adjust_fic=0, analytical_fic=0,
+                                 precision=bnm.PREC_F32, fc_precision=bnm.FC_F32)
+        with bnm.Context(cfg) as c:
+            c.set_sc(W.synthetic_sc(N, 0.9, 1))
+            c.set_noise(bnm.make_noise(1, (T + 1) * 20 * N))
+            c.set_empirical(np.linspace(-0.2, 0.8, bnm.n_pairs(N, False)), np.linspace(-0.5, 1.0, 40))
+            one = np.full((B, N), 0.2)
+            c.set_params(np.full(B, 1.0), one, one, None, one)
+            ms = []
+            for _ in range(3):
+                c.run()
+                assert c.taken_over() == B
+                ms.append(c.timings()["integrate"])
+            took.append(min(ms))
+    print("integration ms", took, flush=True)
+    assert took[1] - took[0] < 300
