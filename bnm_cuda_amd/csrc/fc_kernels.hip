@@ -206,7 +206,7 @@ __device__ void gram_tile(const GramItem& it, int ti, int tj, const int* __restr
             xb[r] = X[kg + (size_t)min(tj * TM + m_of(r), it.M - 1) * it.ldm];
         }
     };
-    load(0);
+    if (it.K > 0) load(0);   // (no pairs within a hemisphere of one node)
     for (int k0 = 0; k0 < it.K; k0 += TK) {
 #pragma unroll
         for (int r = 0; r < RL; ++r) {
