@@ -1,0 +1,60 @@
+"""The row-blocked kernel's builds for more than 512 simulations of 65 to 128 nodes
+(four waves a SIMD, part of the registers spilled), at the smallest and largest node
+counts of each slice length, with FIC restarts.
+
+Bounds: FP32 strict within 1e-6 of the oracle per TR on runs of this length, the same
+FIC trials, wIE to 1e-12; against the build for up to 512 simulations twice that.
+"""
+import numpy as np
+import pytest
+
+import bnm_cuda_amd as bnm
+from bnm_cuda_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+T, TR, I_END, B = 400, 20, 120, 513
+
+
+@pytest.mark.parametrize("N", [65, 80, 81, 100, 104, 105, 128])
+def test_large_population_build(oracle_mod, N):
+    print("case: block kernel, 513 simulations, N", N, flush=True)
+    period = 150 if N % 2 else T + 1
+    rng = np.random.default_rng(N)
+    SC = W.synthetic_sc(N, 0.5, N)
+    G = rng.uniform(0.02, 2.5, B)
+    wEE, wEI = rng.uniform(0.1, 0.4, (B, N)), rng.uniform(0.1, 0.3, (B, N))
+    noise = bnm.make_noise(N, period * 20 * N)
+    emp = rng.uniform(-0.2, 0.8, bnm.n_pairs(N, False)), rng.uniform(-0.5, 1.0, 40)
+    out = {}
+    for n in (B, B - 1):
+        cfg = bnm.default_config(nodes=N, n_sims=n, time_steps=T, bold_tr=TR, n_vols_remove=2, no_fcd=1,
+                                 exc_interhemispheric=0, noise_period_ms=period, max_fic_trials=2, i_sampling_start=20,
+                                 i_sampling_end=I_END, precision=bnm.PREC_F32, kernel=bnm.KERNEL_FAST,
+                                 fc_precision=bnm.FC_F32)
+        with bnm.Context(cfg) as c:
+            c.set_sc(SC)
+            c.set_noise(noise)
+            c.set_empirical(*emp)
+            c.set_params(G[:n], wEE[:n], wEI[:n])
+            c.run()
+            assert c.kernel_name().startswith("block_f32")
+            out[n] = c.outputs()
+    g, small = out[B], out[B - 1]
+    np.testing.assert_array_equal(g["fic_trials"][:-1], small["fic_trials"])
+    assert g["fic_trials"].max() > 0
+    peak = np.abs(g["bold"]).max(axis=(1, 2))
+    assert (np.abs(g["bold"][:-1] - small["bold"]).max(axis=(1, 2)) <= 2e-6 * peak[:-1]).all()
+    some = [0, 100, B - 1]
+    r = oracle_mod.run_simulations(SC, G[some], wEE[some], wEI[some], noise_arr=noise, noise_period_ms=period,
+                                   time_steps=T, bold_tr=TR, n_vols_remove=2, window_size=6, window_step=3,
+                                   emp_fc=emp[0], emp_fcd=emp[1], no_fcd=True, max_fic_trials=2, i_start=20,
+                                   i_end=I_END, exc=False)
+    np.testing.assert_array_equal(g["fic_trials"][some], r["fic_trials"])
+    np.testing.assert_allclose(g["wIE_fic"][some], r["wIE_fic"], rtol=0, atol=1e-12)
+    for i, b in enumerate(some):
+        rel = np.abs(g["bold"][b] - r["bold"][i]).max() / np.abs(r["bold"][i]).max()
+        print("sim", b, "trials", r["fic_trials"][i], "per-TR BOLD rel", rel, flush=True)
+        assert rel <= 1e-6
+    scale = np.abs(r["ext"]).max(axis=(0, 2), keepdims=True)
+    assert (np.abs(g["ext"][some] - r["ext"]) <= 1e-5 * scale).all()
