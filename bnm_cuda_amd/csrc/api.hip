@@ -158,7 +158,7 @@ struct bnm_ctx {
     unsigned long long* gang = nullptr;   // exchange words of kind 10
     int gang_mode = -1, gang_polls = kGangStartPolls, gang_mark = 0;
     bool gang_ran = false;   // the last run was kind 10's
-    int cus = 256;
+    int cus = 256, dev = 0;  // of the device that it was created on
     hipGraphExec_t graph_exec = nullptr;
     bool have_sc = false, have_noise = false, have_emp = false, have_params = false;
     int fast_ls = 0, fast_ks = 0, stream_ks = 0, force_stream = 0, no_ei = 0, ei_ls = 0, ei_bc = 0, ei_form = -1, no_hyb = 0, hyb_ks = 0, hyb_bc = -1, hyb_rr = -1;
@@ -631,11 +631,11 @@ static bnm_ctx* ctx_create(const bnm_config* cfg, int* status, unsigned char* ar
     x->gang_mark = env_int("BNM_GANG_MARK", 0);
     x->hyb_ks = env_int("BNM_HYB_KS", 0);
     {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 0)
+        int v = 0;
+        if (hipGetDevice(&x->dev) == hipSuccess &&
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, x->dev) == hipSuccess && v > 0)
             x->lds_max = (size_t)v;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) x->cus = v;
+        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, x->dev) == hipSuccess && v > 0) x->cus = v;
     }
     x->autotune = c.autotune;
     x->tune_ms = env_int("BNM_TUNE_MS", 300);
@@ -1622,7 +1622,11 @@ static int to_host(bnm_ctx* x, const void* src, size_t bytes, size_t unit, void*
             x->stage = nullptr;
         }
     }
-    bool staged = nt >= 2 && piece && !x->arena && x->stage;
+    // (events and streams that work together have one device: the context's, whatever
+    // the caller's current one is)
+    int dev = x->dev;
+    bool staged = nt >= 2 && piece && !x->arena && x->stage && hipGetDevice(&dev) == hipSuccess;
+    if (staged && dev != x->dev) staged = hipSetDevice(x->dev) == hipSuccess;
     for (int t = 0; t < nt && staged; ++t)
         if (!x->stage_ev[t] && hipEventCreateWithFlags(&x->stage_ev[t], hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
@@ -1631,6 +1635,7 @@ static int to_host(bnm_ctx* x, const void* src, size_t bytes, size_t unit, void*
         }
     if (!staged) {
         lock.unlock();
+        if (dev != x->dev) (void)hipSetDevice(dev);
         if (plain) {
             HIPCHK(hipMemcpy(plain, src, bytes, hipMemcpyDeviceToHost));
             return BNM_OK;
@@ -1640,13 +1645,11 @@ static int to_host(bnm_ctx* x, const void* src, size_t bytes, size_t unit, void*
         f(t.data(), 0, bytes);
         return BNM_OK;
     }
-    int dev = 0;
-    HIPCHK(hipGetDevice(&dev));
     std::atomic<size_t> next{0};
     std::atomic<int> err{(int)hipSuccess};
     auto work = [&](int t) {
         char* slot = x->stage + t * kStageBytes;
-        hipError_t e = t ? hipSetDevice(dev) : hipSuccess;
+        hipError_t e = t ? hipSetDevice(x->dev) : hipSuccess;
         while (e == hipSuccess) {
             const size_t o = next.fetch_add(piece);
             if (o >= bytes) return;
@@ -1665,6 +1668,7 @@ static int to_host(bnm_ctx* x, const void* src, size_t bytes, size_t unit, void*
     }
     work(0);
     for (auto& th : pool) th.join();
+    if (dev != x->dev) (void)hipSetDevice(dev);
     HIPCHK((hipError_t)err.load());
     return BNM_OK;
 }
