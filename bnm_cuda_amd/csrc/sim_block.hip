@@ -48,8 +48,8 @@ __device__ __forceinline__ int block_row(int q, int r) {
 
 }  // namespace
 
-template <class T, int R, int KC, int MAXT, int WAVES>
-__global__ __launch_bounds__(MAXT, WAVES) void k_sim_block(const T* __restrict__ SC, SimArgs a, int SS) {
+template <class T, int R, int KC>
+__device__ __forceinline__ void block_run(const T* __restrict__ SC, const SimArgs& a, int SS) {
     constexpr int Q = 2 * R;                       // lanes of a group, k-slices
     constexpr int VW = 16 / sizeof(T);
     typedef T vec __attribute__((ext_vector_type(VW)));
@@ -229,6 +229,17 @@ __global__ __launch_bounds__(MAXT, WAVES) void k_sim_block(const T* __restrict__
     }
 }
 
+template <class T, int R, int KC, int MAXT, int WAVES>
+__global__ __launch_bounds__(MAXT, WAVES) void k_sim_block(const T* __restrict__ SC, SimArgs a, int SS) {
+    block_run<T, R, KC>(SC, a, SS);
+}
+// no more than MOST waves a SIMD
+template <class T, int R, int KC, int MAXT, int MOST>
+__global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(MOST, MOST))) void k_sim_block_most(
+    const T* __restrict__ SC, SimArgs a, int SS) {
+    block_run<T, R, KC>(SC, a, SS);
+}
+
 // KC: slice lengths that the kernel is built for; R = 4 rows a lane.  FP64 takes
 // up to 128 nodes (16 values x 4 rows = 128 VGPRs); FP32 up to 256, with two
 // waves a SIMD from 129 on.
@@ -262,8 +273,22 @@ static void launch_block_w(const T* SC, const SimArgs& a, const BlockShape& s, h
 // one without spills takes, in cycles a substep, N = 41: 527 / 537 at 128
 // simulations, 1097 / 1403 at 2048; N = 64: 555 / 575 and 1195 / 1488; N = 100:
 // 698 / 677, 844 / 822 at 512, 1436 / 1602 at 1024, 2657 / 3068 at 2048.
+// Where the population (N <= 64) comes to more than half of a second or third wave a
+// SIMD, a build that leaves no room for another: behind other kernels the dispatcher has
+// put one more on some SIMDs and one less on others.  300 ms of 64 nodes, 769 / 900 / 1024
+// simulations behind the analytical FIC: 1.22 / 1.25 / 1.27 ms, 0.93 / 0.95 / 0.99 with
+// it (E/I kernel: 1.02 / 1.03 / 1.05); 32 nodes, 3000: 1.29, 1.07
+// (1.10).  Where the deal is even it costs up to 3 %.
 template <class T, int KC>
 static void launch_block(const T* SC, const SimArgs& a, const BlockShape& s, hipStream_t st) {
+    if constexpr (sizeof(T) == 4 && KC <= 8) {
+        const int waves = a.B * (s.threads / 64), per = (waves + 1023) / 1024;   // per SIMD
+        if (2 * waves > 2048 * per - 1024 && (per == 2 || per == 3)) {
+            if (per == 2) hipLaunchKernelGGL((k_sim_block_most<T, 4, KC, 128, 2>), dim3(a.B), dim3(s.threads), s.smem, st, SC, a, s.SS);
+            else hipLaunchKernelGGL((k_sim_block_most<T, 4, KC, 128, 3>), dim3(a.B), dim3(s.threads), s.smem, st, SC, a, s.SS);
+            return;
+        }
+    }
     if constexpr (sizeof(T) == 4 && KC <= 8) {
         launch_block_w<T, KC, 4>(SC, a, s, st);
     } else if constexpr (sizeof(T) == 4 && KC <= 16) {
