@@ -351,6 +351,43 @@ int fin(bnm_mlp* m, const FusedNet& n, int mode, float lr = 0, float b1 = 0, flo
     return BNM_OK;
 }
 
+// Many rows through a small network go layer by layer: the row blocks' workgroups cost
+// the same whatever the width and come in several rounds, while a layer's product has no
+// weights to wait for.  Same bits either way.  Predictions of 5 -> hidden x depth -> 1,
+// row blocks / layer by layer, ms a call:
+//   BF16   32 x 2:  16384 rows 0.060 / 0.065   32768 0.092 / 0.083   65536 0.166 / 0.126
+//          64 x 4:                                   0.109 / 0.132         0.203 / 0.182
+//         128 x 4:                                   0.121 / 0.173         0.227 / 0.260
+//   FP32   32 x 2:   8192 rows 0.049 / 0.057   16384 0.069 / 0.067   65536 0.205 / 0.131
+//         128 x 4:  16384 rows 0.113 / 0.143   32768 0.198 / 0.182         0.376 / 0.281
+//         256 x 2:                                   0.183 / 0.193         0.348 / 0.327
+//         256 x 4:                                   0.304 / 0.352         0.579 / 0.662
+long weights_of(const bnm_mlp* m) {
+    long w = 0;
+    for (int l = 0; l <= m->depth; ++l) w += (long)m->dims[l] * m->dims[l + 1];
+    return w;
+}
+bool predict_by_layers(const bnm_mlp* m, int rows) {
+    const long w = weights_of(m), L = m->depth + 1;
+    const int h = *std::max_element(m->dims.begin(), m->dims.end());
+    if (m->bf16) return h <= 128 && w < 32768 && rows > 12288 + 4096 * L + 64 * h;
+    return w < 131072 && rows > 8192 + 2048 * L + 64 * h + (h > 128 ? w / 4 : 0);
+}
+// Gradients only through one narrow hidden layer, where the derivatives that the row
+// blocks keep are more than the activations of a layer (8 nodes: 131072 rows 0.63 / 0.66
+// ms, 1000000 5.5 / 4.2; 64 nodes, FP32: 131072 0.79 / 0.90, 262144 1.81 / 1.64).
+bool gradient_by_layers(const bnm_mlp* m, int rows) {
+    const int h = *std::max_element(m->dims.begin(), m->dims.end());
+    return m->depth == 1 && (m->bf16 ? h <= 32 && rows >= 327680 : h <= 64 && rows >= 229376);
+}
+// ... and those whose buffers are not to be had
+bool gradient_fused(bnm_mlp* m, int rows) {
+    if (!m->fused || gradient_by_layers(m, rows)) return false;
+    if (ensure_fused(m, rows) == BNM_OK) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 // Partial sums of the loss that a gradient over `rows` rows leaves.
 int loss_parts(const bnm_mlp* m, int rows) {
     const int R = block_rows(m, rows);
@@ -581,7 +618,7 @@ int bnm_mlp_set_params(bnm_mlp* m, const float* in) {
 int bnm_mlp_predict(bnm_mlp* m, const float* X, int n, float* Y) {
     if (!m || !X || !Y || n < 1) return BNM_E_ARG;
     const int chunk = kChunk;
-    if (m->fused) {
+    if (m->fused && !predict_by_layers(m, std::min(n, chunk))) {
         int e = ensure_floats(&m->px, &m->xcap, std::min(n, chunk), m->in + m->out);
         if (e) return e;
         FusedNet f = m->net;
@@ -616,9 +653,8 @@ int bnm_mlp_predict(bnm_mlp* m, const float* X, int n, float* Y) {
 int bnm_mlp_loss_grad(bnm_mlp* m, const float* X, const float* T, int n, float* loss, float* grad) {
     if (!m || !X || !T || n < 1) return BNM_E_ARG;
     int e = 0;
-    if (m->fused) {
+    if (gradient_fused(m, n)) {
         const int parts = loss_parts(m, n);
-        if ((e = ensure_fused(m, n))) return e;
         if ((e = ensure_floats(&m->px, &m->xcap, n, m->in + m->out))) return e;
         if ((e = ensure_floats(&m->loss_part, &m->loss_cap, parts, 1))) return e;
         FusedNet f = m->net;
@@ -673,9 +709,10 @@ int bnm_mlp_set_data(bnm_mlp* m, const float* X, const float* T, int n) {
 int bnm_mlp_train(bnm_mlp* m, int epochs, int batch, float lr, unsigned seed, float* loss) {
     if (!m || m->n_data < 1 || batch < 1 || epochs < 1) return BNM_E_ARG;
     batch = std::min(batch, m->n_data);
-    int e = m->fused ? ensure_fused(m, batch) : ensure_rows(m, batch);
+    const bool fused = gradient_fused(m, batch);
+    int e = fused ? BNM_OK : ensure_rows(m, batch);
     if (e) return e;
-    const int parts = m->fused ? loss_parts(m, batch) : kLossBlocks;
+    const int parts = fused ? loss_parts(m, batch) : kLossBlocks;
     if ((e = ensure_floats(&m->loss_part, &m->loss_cap, parts, 1))) return e;
     if (m->idx_cap < m->n_data) {
         if (m->idx) { (void)hipFree(m->idx); m->idx = nullptr; }
@@ -697,7 +734,7 @@ int bnm_mlp_train(bnm_mlp* m, int epochs, int batch, float lr, unsigned seed, fl
         hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(64), 0, m->st, m->loss_part, parts, 0.0f);
         for (int b = 0; b < nb; ++b) {
             const int* ib = m->idx + (long)b * batch;
-            if (m->fused) {
+            if (fused) {
                 FusedNet f = m->net;
                 f.rows = batch;
                 f.X = m->X;
@@ -720,6 +757,8 @@ int bnm_mlp_train(bnm_mlp* m, int epochs, int batch, float lr, unsigned seed, fl
                                b2, eps, c1, c2);
         }
         MCHK(hipGetLastError());
+        // the row blocks' copies of the weights
+        if (m->fused && !fused && (e = fin(m, m->net, 0))) return e;
         if (loss) {
             MCHK(hipMemcpyAsync(lp.data(), m->loss_part, parts * sizeof(float), hipMemcpyDeviceToHost, m->st));
             MCHK(hipStreamSynchronize(m->st));
