@@ -1031,9 +1031,10 @@ static std::vector<Variant> candidates(const bnm_ctx* x) {
     // several workgroups per simulation: where it pays depends on the population
     // (N = 400, FP32: 0.7 us a substep on seven CUs against 2.6 on one), so it
     // is for the tuner to say
-    if (c.kernel == BNM_KERNEL_AUTO && (x->autotune || x->gang_mode > 0) && !switched) {
+    if (c.kernel == BNM_KERNEL_AUTO && (x->autotune || x->gang_mode > 0) && !switched && x->gang) {
         // (the tuner's order: what is likely best first, see choose_variant; the
-        // streaming kernels are left out where a hybrid one applies)
+        // streaming kernels are left out where a hybrid one applies: to 512 nodes they
+        // never win, beyond they do, N = 1000, FP32, 48.4 ms against 53.5)
         bool hyb = false;
         for (const Variant& v : out) hyb = hyb || v.kind == 5 || v.kind == 7;
         if (hyb) out.erase(std::remove_if(out.begin(), out.end(), [](const Variant& v) { return v.kind == 1; }), out.end());
