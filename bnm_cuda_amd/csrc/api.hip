@@ -956,11 +956,8 @@ static std::vector<Variant> candidates(const bnm_ctx* x) {
     // unless a switch asks for one of the others: it is faster than every split
     // and E/I shape (N = 100, 128 simulations, per substep: FP32 0.28 us against
     // 0.38, FP64 0.32 against 0.72) and than the streaming and hybrid kernels.
-    // Timed against it are the MFMA kernel and the E/I and split kernels (large
-    // populations) and, for N > 128, the sparse kernel (SCs of low density).  For up
-    // to 16 nodes the strict E/I kernel stands in for it in FP32, the faster one to
-    // 2048 simulations (one wave either way; 400 ms of 10 nodes, 1 / 1024 / 2048
-    // simulations: 0.65 / 0.67 / 0.89 ms against 0.69 / 0.73 / 0.96); beyond, both.
+    // Timed against it are the MFMA kernel (large populations) and, for N > 128,
+    // the sparse kernel (SCs of low density).
     const bool switched = x->no_ei || x->ei_form >= 0 || x->ei_bc || x->force_stream || x->stream_ks > 0 ||
                           x->no_hyb || x->hyb_bc >= 0 || x->hyb_rr >= 0 || x->no_sparse;
     if (!switched) {
@@ -973,10 +970,6 @@ static std::vector<Variant> candidates(const bnm_ctx* x) {
                 // (large populations of few nodes are a matter of instructions per
                 // simulation, not of latency: both pools in one lane, one wave for
                 // 64 nodes, 1.17 ms against 1.62 at N = 41, 2036 simulations)
-                if (x->N <= 16 && x->autotune && variant_ok(x, {4, 2, 1, 3 | 64})) {
-                    out[0] = {4, 2, 1, 3 | 64};
-                    if (x->B > 2048) add({9, 1, 1, 0});
-                }
                 if (x->B > 512) add({0, 1, 1, 0});
                 add({2, 0, 0, 0});
             }

@@ -1,7 +1,7 @@
 """The row-blocked kernel's builds for more than 512 simulations of 65 to 128 nodes
 (four waves a SIMD, part of the registers spilled) and those for no more than two or three
 waves a SIMD (up to 64 nodes), at the smallest and largest node counts of each slice
-length, with FIC restarts; and the tuner's choice for up to 16 nodes.
+length, with FIC restarts.
 
 Bounds: FP32 strict within 1e-6 of the oracle per TR on runs of 2.5 s, the same FIC
 trials, wIE to 1e-12; against the build for smaller populations twice that.
@@ -62,32 +62,3 @@ def test_large_population_build(oracle_mod, N, B):
         assert rel <= 1e-6
     scale = np.abs(r["ext"]).max(axis=(0, 2), keepdims=True)
     assert (np.abs(g["ext"][some] - r["ext"]) <= 1e-5 * scale).all()
-
-
-@pytest.mark.parametrize("N", [2, 9, 16])
-def test_tuned_kernel_for_few_nodes(oracle_mod, N):
-    """AUTO times the strict E/I kernel in the row-blocked one's place: the same bound."""
-    print("case: tuned kernel, N", N, flush=True)
-    B = 5
-    rng = np.random.default_rng(N)
-    SC = W.synthetic_sc(N, 0.9, N)
-    G, wEE, wEI = rng.uniform(0.5, 2.5, B), rng.uniform(0.1, 0.4, (B, N)), rng.uniform(0.1, 0.3, (B, N))
-    noise = bnm.make_noise(N, (T + 1) * 20 * N)
-    emp = rng.uniform(-0.2, 0.8, bnm.n_pairs(N, False)), rng.uniform(-0.5, 1.0, 40)
-    kw = dict(time_steps=T, bold_tr=TR, n_vols_remove=2, max_fic_trials=2, noise_period_ms=T + 1)
-    cfg = bnm.default_config(nodes=N, n_sims=B, no_fcd=1, exc_interhemispheric=0, i_sampling_start=200,
-                             i_sampling_end=I_END, precision=bnm.PREC_F32, fc_precision=bnm.FC_F32, **kw)
-    with bnm.Context(cfg) as c:
-        c.set_sc(SC)
-        c.set_noise(noise)
-        c.set_empirical(*emp)
-        c.set_params(G, wEE, wEI)
-        c.run()
-        assert c.kernel_name().startswith("split_ei_f32") and "strict" in c.kernel_name()
-        assert "block_f32" not in c.tune_log()
-        g = c.outputs()
-    r = oracle_mod.run_simulations(SC, G, wEE, wEI, noise_arr=noise, window_size=6, window_step=3, emp_fc=emp[0],
-                                   emp_fcd=emp[1], no_fcd=True, i_start=200, i_end=I_END, exc=False, **kw)
-    np.testing.assert_array_equal(g["fic_trials"], r["fic_trials"])
-    for b in range(B):
-        assert np.abs(g["bold"][b] - r["bold"][b]).max() <= 1e-6 * np.abs(r["bold"][b]).max()
