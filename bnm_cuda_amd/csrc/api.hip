@@ -956,8 +956,8 @@ static std::vector<Variant> candidates(const bnm_ctx* x) {
     // unless a switch asks for one of the others: it is faster than every split
     // and E/I shape (N = 100, 128 simulations, per substep: FP32 0.28 us against
     // 0.38, FP64 0.32 against 0.72) and than the streaming and hybrid kernels.
-    // Timed against it are the MFMA kernel (large populations) and, for N > 128,
-    // the sparse kernel (SCs of low density).
+    // Timed against it are the MFMA, split and E/I kernels (large populations) and,
+    // for N > 128, the sparse kernel (SCs of low density).
     const bool switched = x->no_ei || x->ei_form >= 0 || x->ei_bc || x->force_stream || x->stream_ks > 0 ||
                           x->no_hyb || x->hyb_bc >= 0 || x->hyb_rr >= 0 || x->no_sparse;
     if (!switched) {
@@ -970,6 +970,11 @@ static std::vector<Variant> candidates(const bnm_ctx* x) {
                 // (large populations of few nodes are a matter of instructions per
                 // simulation, not of latency: both pools in one lane, one wave for
                 // 64 nodes, 1.17 ms against 1.62 at N = 41, 2036 simulations)
+                // (up to 16 nodes the strict E/I kernel takes fewer instructions: 2 s of 10
+                // nodes, 2048 simulations 4.32 ms against 4.61, 3000 7.50 against 6.39; to
+                // 1024 simulations, where latency counts, it is 5 % faster on short runs and
+                // 3 % slower once the noise comes from memory)
+                if (x->N <= 16 && x->B > 1024) add({4, 2, 1, 3 | 64});
                 if (x->B > 512) add({0, 1, 1, 0});
                 add({2, 0, 0, 0});
             }
