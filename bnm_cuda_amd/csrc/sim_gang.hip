@@ -23,7 +23,7 @@
 // wait for its noise from HBM first.
 //
 // Waiting: members start when all are there and on one XCD.  A member that waits
-// in vain (GangArgs::start_polls, 1.5 s: another kernel holds the CUs) marks the
+// in vain (GangArgs::start_polls, 1.6 s: another kernel holds the CUs) marks the
 // simulation, and tells the rest of the launch, whose members then wait no more: those
 // that do not find all the others there mark at once, so a launch waits once.  It waits
 // that long because the CUs mostly come free: two contexts of 32 simulations of N = 400,
@@ -37,7 +37,7 @@
 // as many groups as have a CU for each member: members of a second round of
 // workgroups would start one by one, as simulations of the first end, and wait in
 // vain for each other (FP64, 128 simulations of N = 400 with FIC, 2.7 s: 0.64 s with
-// the launch that takes over, 0.48 on one workgroup each, 0.22 with groups).
+// the hybrid kernel behind them, 0.48 on that alone, 0.22 with groups).
 //
 // What bounds it: the exchange.  At N = 400 (FP32, 16 simulations on 112 CUs) one
 // substep is 1810 cycles: 850 from store to the value in the others' LDS, 450 of
