@@ -1134,12 +1134,15 @@ static int choose_variant(bnm_ctx* x) {
 // analyze_only: FC, FCD and fit of the BOLD already in the context (no FIC
 // initialisation, no integration, no FIC penalty)
 // solo: with one workgroup per simulation (several contexts in one graph)
-static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only = false, bool solo = false) {
+// ready: recorded when the integration is the next to start
+static int enqueue_run(bnm_ctx* x, hipStream_t st, bool timed, bool analyze_only = false, bool solo = false,
+                       hipEvent_t ready = nullptr) {
     const bnm_config& c = x->cfg;
     if (timed) HIPCHK(hipEventRecord(x->ev[0], st));
     if (c.do_fic && c.analytical_fic && !analyze_only)
         HIPCHK(launch_fic_analytical(x->SC64, x->N, x->B, x->G, x->wEE, x->wEI, x->wIEfic,
                                      x->unstable, st));
+    if (ready) HIPCHK(hipEventRecord(ready, st));
     if (timed) HIPCHK(hipEventRecord(x->ev[1], st));
     if (!analyze_only) {
         const SimArgs a = make_args(x);
@@ -1420,7 +1423,11 @@ static bool small_workgroup(const bnm_ctx* x) {
             const SparseShape s = sparse_shape(x->N, x->sp_P[v.ls - 1], v.ls, x->lds_max, el);
             threads = s.threads; smem = s.smem; break;
         }
-        case 9: { const BlockShape s = block_shape(x->N, el); threads = s.threads; smem = s.smem; break; }
+        case 9: {
+            if (x->f64 && x->N > 64) return false;   // (more than half of a SIMD's registers)
+            const BlockShape s = block_shape(x->N, el);
+            threads = s.threads; smem = s.smem; break;
+        }
         default: threads = ((x->N + 63) / 64) * 64; smem = (size_t)x->N * el; break;
     }
     return threads <= 256 && smem <= 32 * 1024;
@@ -1454,11 +1461,11 @@ bnm_multi* bnm_multi_create(bnm_ctx** ctxs, int n, int* status) {
     // the longest one down.  K = CUs / (largest workgroup count) branches run
     // concurrently; contexts go to branches longest first, each to the branch
     // with the least estimated work (LPT), and run one after another within
-    // it, except that two consecutive contexts with small workgroups
-    // (small_workgroup) run side by side on the CUs the branch holds (with
-    // 2K branches of CU-filling kernels that means: after the large context
-    // before them).  BNM_MULTI_BRANCHES overrides K (n: every context its own
-    // branch).
+    // it, except that two contexts with small workgroups (small_workgroup),
+    // consecutive ones or paired beforehand, run side by side on the CUs the
+    // branch holds (with 2K branches of CU-filling kernels that means: after
+    // the large context before them).  BNM_MULTI_BRANCHES overrides K (n:
+    // every context its own branch).
     int cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
@@ -1476,29 +1483,67 @@ bnm_multi* bnm_multi_create(bnm_ctx** ctxs, int n, int* status) {
     std::vector<int> order(n);
     for (int i = 0; i < n; ++i) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return est[a] > est[b]; });
-    std::vector<std::vector<int>> branch(K);
-    std::vector<double> load(K, 0.0);
-    for (int i : order) {
-        int b = 0;
-        for (int q = 1; q < K; ++q)
-            if (load[q] < load[b]) b = q;
-        branch[b].push_back(i);
-        load[b] += est[i];
-    }
+    std::vector<char> small(n);
+    for (int i = 0; i < n; ++i) small[i] = small_workgroup(m->ctxs[i]);
     // stages of each branch: one context, or two small ones side by side
-    std::vector<std::vector<std::vector<int>>> stages(K);
-    for (int b = 0; b < K; ++b) {
-        const auto& br = branch[b];
-        for (size_t q = 0; q < br.size(); ++q) {
-            if (q + 1 < br.size() && small_workgroup(m->ctxs[br[q]]) && small_workgroup(m->ctxs[br[q + 1]])) {
-                stages[b].push_back({br[q], br[q + 1]});
-                ++q;
-            } else {
-                stages[b].push_back({br[q]});
-            }
+    typedef std::vector<std::vector<std::vector<int>>> Stages;
+    std::vector<double> load;
+    auto cost = [&](const std::vector<int>& st) { return st.size() == 2 ? std::max(est[st[0]], est[st[1]]) : est[st[0]]; };
+    auto longest = [&](const Stages& s) {
+        double t = 0;
+        for (const auto& br : s) {
+            double v = 0;
+            for (const auto& st : br) v += cost(st);
+            t = std::max(t, v);
         }
+        return t;
+    };
+    auto least = [&](const std::vector<double>& v) { return (int)(std::min_element(v.begin(), v.end()) - v.begin()); };
+    Stages stages(K);
+    {
+        std::vector<std::vector<int>> branch(K);
+        load.assign(K, 0.0);
+        for (int i : order) {
+            const int q = least(load);
+            branch[q].push_back(i);
+            load[q] += est[i];
+        }
+        for (int b = 0; b < K; ++b)
+            for (size_t q = 0; q < branch[b].size(); ++q) {
+                const int i = branch[b][q];
+                stages[b].push_back({i});
+                if (q + 1 < branch[b].size() && small[i] && small[branch[b][q + 1]]) stages[b].back().push_back(branch[b][++q]);
+            }
+    }
+    // ... or the small ones paired first, where that ends sooner (FP32, 128 simulations
+    // each of N = 100 and 68, 6 s, and of N = 200, 3 s: 17, 16 and 14 ms; paired after
+    // the deal, 68 and 200 in turn beside 100, 32 ms, paired before it 19)
+    {
+        std::vector<std::vector<int>> units;
+        int open = -1;                          // unit with one small context
+        for (int i : order) {
+            if (small[i] && open >= 0) {
+                units[open].push_back(i);
+                open = -1;
+                continue;
+            }
+            if (small[i]) open = (int)units.size();
+            units.push_back({i});
+        }
+        std::stable_sort(units.begin(), units.end(),
+                         [&](const std::vector<int>& a, const std::vector<int>& b) { return cost(a) > cost(b); });
+        Stages paired(K);
+        std::vector<double> v(K, 0.0);
+        for (const auto& u : units) {
+            const int q = least(v);
+            paired[q].push_back(u);
+            v[q] += cost(u);
+        }
+        if ((int)units.size() >= K && longest(paired) < 0.95 * longest(stages)) stages = paired;
+    }
+    for (int b = 0; b < K; ++b) {
         load[b] = 0;
-        for (const auto& st : stages[b]) load[b] += st.size() == 2 ? std::max(est[st[0]], est[st[1]]) : est[st[0]];
+        for (const auto& st : stages[b]) load[b] += cost(st);
     }
     {
         char buf[96];
@@ -1525,23 +1570,41 @@ bnm_multi* bnm_multi_create(bnm_ctx** ctxs, int n, int* status) {
     int r = BNM_OK;
     hipError_t e = hipEventRecord(m->fork, s0);
     std::vector<hipStream_t> bst(K);
-    for (int b = 0; b < K; ++b) bst[b] = m->ctxs[branch[b][0]]->st;
+    for (int b = 0; b < K; ++b) bst[b] = m->ctxs[stages[b][0][0]]->st;
     for (int b = 0; b < K && e == hipSuccess; ++b)
         if (bst[b] != s0) e = hipStreamWaitEvent(bst[b], m->fork, 0);
-    for (int b = 0; b < K && e == hipSuccess && !r; ++b)
+    // Branches that begin with a small context begin when the others' first
+    // integrations are about to: workgroups that fill a CU find none empty once
+    // the small ones lie on all of them (the three populations above: 29 ms).
+    auto new_event = [&]() {
+        hipEvent_t v = nullptr;
+        e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+        if (e == hipSuccess) m->pair_events.push_back(v);
+        return v;
+    };
+    std::vector<int> turn(K);
+    for (int b = 0; b < K; ++b) turn[b] = b;
+    std::stable_partition(turn.begin(), turn.end(), [&](int b) { return !small[stages[b][0][0]]; });
+    std::vector<hipEvent_t> begun;
+    for (int b : turn) {
+        const bool large = !small[stages[b][0][0]];
+        if (!large)
+            for (hipEvent_t v : begun)
+                if (e == hipSuccess) e = hipStreamWaitEvent(bst[b], v, 0);
         for (const auto& st : stages[b]) {
             if (r || e != hipSuccess) break;
             if (st.size() == 1) {
-                r = enqueue_run(m->ctxs[st[0]], bst[b], false, false, true);
+                hipEvent_t v = nullptr;
+                if (large && &st == &stages[b][0]) {
+                    v = new_event();
+                    if (e == hipSuccess) begun.push_back(v);
+                }
+                if (e == hipSuccess) r = enqueue_run(m->ctxs[st[0]], bst[b], false, false, true, v);
                 continue;
             }
             // the second context on its own stream, forked from and joined to
             // the branch's stream around the first
-            hipEvent_t f = nullptr, jn = nullptr;
-            e = hipEventCreateWithFlags(&f, hipEventDisableTiming);
-            if (e == hipSuccess) m->pair_events.push_back(f);
-            if (e == hipSuccess) e = hipEventCreateWithFlags(&jn, hipEventDisableTiming);
-            if (e == hipSuccess) m->pair_events.push_back(jn);
+            const hipEvent_t f = new_event(), jn = e == hipSuccess ? new_event() : nullptr;
             hipStream_t s2 = m->ctxs[st[1]]->st;
             if (e == hipSuccess) e = hipEventRecord(f, bst[b]);
             if (e == hipSuccess) e = hipStreamWaitEvent(s2, f, 0);
@@ -1550,6 +1613,7 @@ bnm_multi* bnm_multi_create(bnm_ctx** ctxs, int n, int* status) {
             if (e == hipSuccess && !r) e = hipEventRecord(jn, s2);
             if (e == hipSuccess && !r) e = hipStreamWaitEvent(bst[b], jn, 0);
         }
+    }
     for (int b = 0; b < K && e == hipSuccess && !r; ++b) {
         if (bst[b] == s0) continue;
         e = hipEventRecord(m->joins[b], bst[b]);
